@@ -214,6 +214,31 @@ def test_row_norm_vs_reference(gpu, mode, adds, dim_actual, H):
     assert ((out.double().cpu() - ref).abs() <= 1e-2 * ref.abs().clamp_min(1)).all()
 
 
+@pytest.mark.parametrize("H", [8, 2048, 2056, 4096, 4104, 8192, 8200, 16384, 16392])
+@pytest.mark.parametrize("mode", [1, 2])
+def test_row_norm_chunk_counts(gpu, mode, H):
+    """Rows at the edges of the compiled chunk counts (256 threads x 1, 2, 4
+    or 8 chunks of 8 elements; 16392 takes the element path), gamma starting
+    at an odd float, adds in a padded row stride.  The result is one bf16
+    rounding (2^-8 of the value) of fp32 math whose relative error is far
+    below it."""
+    rows, pad = 3, 8
+    g = torch.Generator().manual_seed(H + mode)
+    wide = lambda: torch.randn(rows, H + pad, generator=g).to(bf).to(gpu)[:, :H]
+    x, a0, a1 = wide(), wide(), wide()
+    gam = (torch.rand(H + 1, generator=g) + 0.5).to(gpu)[1:]
+    bet = torch.randn(H + 1, generator=g).to(gpu)[1:] if mode == 2 else None
+    out = K.row_norm(x, mode, 1e-5, gam, bet, add0=a0, add1=a1)
+    xs = ((x + a0) + a1).double()
+    if mode == 1:
+        ref = xs * torch.rsqrt(xs.pow(2).mean(-1, keepdim=True) + 1e-5) * gam.double()
+    else:
+        mu = xs.mean(-1, keepdim=True)
+        ref = (xs - mu) * torch.rsqrt(xs.var(-1, keepdim=True, unbiased=False) + 1e-5) \
+            * gam.double() + bet.double()
+    assert ((out.double() - ref).abs() <= 2 ** -8 * ref.abs() + 1e-5).all()
+
+
 QKV_CASES = [
     # norm, adds, bias, rope (None / "bf16" / "f32"), qk norms, layout
     ("none", False, True, "f32", False, "BSD"),

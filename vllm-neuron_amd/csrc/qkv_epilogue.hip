@@ -327,36 +327,69 @@ __global__ __launch_bounds__(256) void row_norm_kernel(mia_row_norm_args a) {
 
 // Vector path: dim % 8 == 0, rows 16-byte aligned, at most 256 * kRowChunks
 // chunks of 8 elements per row.  The row stays in registers (8 floats per
-// chunk), so it is read once and written once, 16 bytes per access.
+// chunk), so it is read once and written once, 16 bytes per access.  NC is
+// the chunks of a thread: every chunk's loads (clamped into the row) are
+// issued before the first is used, and with few chunks gamma is loaded before
+// the reduction too, so a row costs one memory round trip, the reduction and
+// the store.  Bound by HBM and that latency: 2048 x 4096 rows (33.6 MB) take
+// 6.7-7.7 us (4.4-5.0 TB/s); one kernel for 1 to 8 chunks, which tested and
+// loaded each chunk in turn and packed bf16 in integer code, took 24.0.
 constexpr int kRowChunks = 8;
+// gamma may start at any float: a 16-byte load that only needs dword alignment
+typedef f32x4_t f32x4_dword_t __attribute__((aligned(4)));
 
+template <int NC>
 __global__ __launch_bounds__(256) void row_norm_vec_kernel(mia_row_norm_args a) {
+  constexpr bool kEarlyGamma = NC <= 2;
   __shared__ float red[2][4];
   const int64_t row = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int nch = a.dim / 8;
-  auto chunk = [&](const void *base, int c) {
-    return *reinterpret_cast<const u32x4_t *>((const uint16_t *)base + row * a.in_stride + 8 * c);
+  const int64_t at = row * a.in_stride;
+  int col[NC];
+#pragma unroll
+  for (int k = 0; k < NC; ++k) col[k] = 8 * (tid + 256 * k < nch ? tid + 256 * k : 0);
+  auto load = [&](const void *base, u32x4_t *w) {
+#pragma unroll
+    for (int k = 0; k < NC; ++k)
+      w[k] = *reinterpret_cast<const u32x4_t *>((const uint16_t *)base + at + col[k]);
   };
-  float v[kRowChunks][8];
+  auto load_vec = [&](const float *p, f32x4_t (*w)[2]) {
+#pragma unroll
+    for (int k = 0; k < NC; ++k) {
+      w[k][0] = *reinterpret_cast<const f32x4_dword_t *>(p + col[k]);
+      w[k][1] = *reinterpret_cast<const f32x4_dword_t *>(p + col[k] + 4);
+    }
+  };
+  u32x4_t w0[NC];
+  load(a.in, w0);
+  f32x4_t g[NC][2];
+  if (kEarlyGamma && a.gamma) load_vec(a.gamma, g);
+  float v[NC][8];
+#pragma unroll
+  for (int k = 0; k < NC; ++k)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[k][e] = (e & 1) ? bf16hi(w0[k][e >> 1]) : bf16lo(w0[k][e >> 1]);
+  auto add = [&](const void *base) {
+    u32x4_t w[NC];
+    load(base, w);
+#pragma unroll
+    for (int k = 0; k < NC; ++k)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const uint32_t r = pack2_bf16(v[k][2 * q] + bf16lo(w[k][q]), v[k][2 * q + 1] + bf16hi(w[k][q]));
+        v[k][2 * q] = bf16lo(r);
+        v[k][2 * q + 1] = bf16hi(r);
+      }
+  };
+  if (a.add0) add(a.add0);
+  if (a.add1) add(a.add1);
   float s = 0.f;
 #pragma unroll
-  for (int k = 0; k < kRowChunks; ++k) {
-    const int c = tid + 256 * k;
-    if (c >= nch) break;
-    const u32x4_t w0 = chunk(a.in, c);
-    u32x4_t w1 = {0u, 0u, 0u, 0u}, w2 = {0u, 0u, 0u, 0u};
-    if (a.add0) w1 = chunk(a.add0, c);
-    if (a.add1) w2 = chunk(a.add1, c);
+  for (int k = 0; k < NC; ++k) {
+    if (tid + 256 * k >= nch) break;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int q = e >> 1;
-      float x = (e & 1) ? bf16hi(w0[q]) : bf16lo(w0[q]);
-      if (a.add0) x = round_bf16(x + ((e & 1) ? bf16hi(w1[q]) : bf16lo(w1[q])));
-      if (a.add1) x = round_bf16(x + ((e & 1) ? bf16hi(w2[q]) : bf16lo(w2[q])));
-      v[k][e] = x;
-      s += a.mode == 2 ? x : x * x;
-    }
+    for (int e = 0; e < 8; ++e) s += a.mode == 2 ? v[k][e] : v[k][e] * v[k][e];
   }
   auto block_sum = [&](float x, int slot) {
 #pragma unroll
@@ -370,7 +403,7 @@ __global__ __launch_bounds__(256) void row_norm_vec_kernel(mia_row_norm_args a) 
     const float mean = block_sum(s, 0) / (float)a.dim;
     float q = 0.f;
 #pragma unroll
-    for (int k = 0; k < kRowChunks; ++k) {
+    for (int k = 0; k < NC; ++k) {
       if (tid + 256 * k >= nch) break;
 #pragma unroll
       for (int e = 0; e < 8; ++e) q += (v[k][e] - mean) * (v[k][e] - mean);
@@ -381,21 +414,25 @@ __global__ __launch_bounds__(256) void row_norm_vec_kernel(mia_row_norm_args a) 
     const int n = a.dim_actual > 0 ? a.dim_actual : a.dim;
     scale = 1.0f / sqrtf(block_sum(s, 0) / (float)n + a.eps);
   }
+  if (!kEarlyGamma && a.gamma) load_vec(a.gamma, g);
   uint16_t *out = (uint16_t *)a.out + row * a.out_stride;
 #pragma unroll
-  for (int k = 0; k < kRowChunks; ++k) {
-    const int c = tid + 256 * k;
-    if (c >= nch) break;
-    uint32_t b[8];
+  for (int k = 0; k < NC; ++k) {
+    float y[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      float y = (v[k][e] - shift) * scale;
-      if (a.gamma) y *= a.gamma[8 * c + e];
-      if (a.beta) y += a.beta[8 * c + e];
-      b[e] = f32_to_bf16_bits(y);
+    for (int e = 0; e < 8; ++e) y[e] = (v[k][e] - shift) * scale;
+    if (a.gamma) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) y[e] *= g[k][e >> 2][e & 3];
     }
-    *reinterpret_cast<u32x4_t *>(out + 8 * c) =
-        u32x4_t{b[0] | (b[1] << 16), b[2] | (b[3] << 16), b[4] | (b[5] << 16), b[6] | (b[7] << 16)};
+    if (a.beta) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) y[e] += a.beta[col[k] + e];
+    }
+    if (tid + 256 * k < nch)
+      *reinterpret_cast<u32x4_t *>(out + col[k]) =
+          u32x4_t{pack2_bf16(y[0], y[1]), pack2_bf16(y[2], y[3]), pack2_bf16(y[4], y[5]),
+                  pack2_bf16(y[6], y[7])};
   }
 }
 
@@ -431,10 +468,19 @@ int launch_row_norm(const mia_row_norm_args &a, hipStream_t s) {
   const bool vec = a.dim % 8 == 0 && a.dim / 8 <= 256 * kRowChunks && a.in_stride % 8 == 0 &&
                    a.out_stride % 8 == 0 && al16(a.in) && al16(a.add0) && al16(a.add1) &&
                    al16(a.out);
-  if (vec)
-    hipLaunchKernelGGL(row_norm_vec_kernel, dim3((unsigned)a.rows), dim3(256), 0, s, a);
+  // chunks per thread: the smallest compiled count that holds the row
+  const dim3 grid((unsigned)a.rows), block(256);
+  const int nc = (a.dim / 8 + 255) / 256;
+  if (!vec)
+    hipLaunchKernelGGL(row_norm_kernel, grid, block, 0, s, a);
+  else if (nc <= 1)
+    hipLaunchKernelGGL(row_norm_vec_kernel<1>, grid, block, 0, s, a);
+  else if (nc <= 2)
+    hipLaunchKernelGGL(row_norm_vec_kernel<2>, grid, block, 0, s, a);
+  else if (nc <= 4)
+    hipLaunchKernelGGL(row_norm_vec_kernel<4>, grid, block, 0, s, a);
   else
-    hipLaunchKernelGGL(row_norm_kernel, dim3((unsigned)a.rows), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(row_norm_vec_kernel<8>, grid, block, 0, s, a);
   return check_hip(hipGetLastError(), "row norm launch");
 }
 
