@@ -362,3 +362,38 @@ def test_copy_ring_output_only_8_byte_aligned(gpu, split):
     torch.cuda.synchronize()
     assert torch.equal(view, base)
     assert (wide[:, :, :4] == 7.0).all() and (wide[:, :, 132:] == 7.0).all()
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("bs,new,prior,window,use_sink", [
+    (16, 1, 0, 0, False),        # one row, one key
+    (32, 63, 0, 0, True),        # one partial key tile
+    (64, 64, 64, 0, False),      # rows and keys end on a tile
+    (16, 65, 192, 0, False),     # one key past a tile, the row tile wraps
+    (128, 129, 128, 64, True),   # block wider than a tile, window edge inside one
+    (16, 200, 320, 130, False),
+])
+def test_copy_ring_tile_edges_and_rising_scores(gpu, d, bs, new, prior, window, use_sink):
+    """Row and key counts at the edges of the tiles, with scores that rise by
+    far more than 2^8 between key tiles, so that every row's maximum moves
+    several times.  Score error: q * scale is rounded to bf16 (relative 2^-9,
+    uniform: rms 2^-9 / sqrt 3), which moves a score of standard deviation 4
+    by 4.5e-3 rms, four times that at the tail; it enters the output as a
+    relative error of the probabilities, on top of the 2e-2 that the bf16
+    probabilities and output are allowed."""
+    cfg = W.PrefillConfig("t", 1, 8, 2, d, bs, new, prior, prior, seed=140 + new)
+    b = W.make_prefill_batch(cfg, gpu)
+    K.kv_write(b.k_new, b.v_new, b.slots, b.k_cache, b.v_cache)
+    n = prior + new
+    for t in range(n):  # keys of tile t / 64: standard deviation 0.25, 1, 4, 4, ...
+        blk = int(b.block_table[0, t // bs])
+        b.k_cache[blk, :, t % bs] *= min(4.0, 0.25 * 4.0 ** (t // 64))
+    sink = torch.randn(8, generator=torch.Generator().manual_seed(new)).to(gpu) if use_sink else None
+    out = K.paged_prefill(b.q, b.cu_seqlens, b.prior, new, b.k_cache, b.v_cache, b.block_table,
+                          scale=d ** -0.5, sliding_window=window, sink=sink)
+    ks = _seq_kv(b.k_cache.cpu(), b.block_table[0].cpu(), n, 2)
+    vs = _seq_kv(b.v_cache.cpu(), b.block_table[0].cpu(), n, 2)
+    f = OSg.fp32_prefill(b.q.cpu(), ks, vs, prior, d ** -0.5, window,
+                         None if sink is None else sink.cpu())
+    err = (out.float().cpu().double() - f).abs().max().item()
+    assert err <= TOL_BF16 + 4 * 4.5e-3, err

@@ -130,7 +130,7 @@ MIA_DEV bool row_range(const PrefillKParams &p, int prior, int kvl, int pos, int
   if (p.bmin && row_ok) {
     const int64_t bi = tok * p.b_st + (int64_t)hq * p.b_sh;
     lo = max(lo, p.bmin[bi]);
-    hi = min(hi, p.bmax[bi]);
+    hi = max(min(hi, p.bmax[bi]), 0);
   }
   const bool uni = p.uniform && !p.sink && row_ok && max(lo, 0) >= hi && kvl > 0;
   if (uni) {
@@ -468,29 +468,56 @@ struct RowMax {
   MIA_DEV float final_max() const { return set ? m : -INFINITY; }
 };
 
-// One tile of the online softmax over sacc = s - m (masked keys -inf) of
-// the lane's row: probabilities as bf16 pairs into pk, acc_o rescaled when
-// the maximum moves, returns the updated partial sum of the lane.
-// Lazy rescaling: the maximum only moves when a score exceeds it by more
-// than 8 (log2 units), so probabilities stay below 2^8 and the accumulators
-// are rescaled only on such tiles; the first visible key of a row always
-// sets it.  The sum adds the bf16-rounded probabilities the PV product uses
-// (v_dot2c_f32_bf16 with (1, 1)).
-template <int DBLK>
-MIA_DEV float softmax_tile(f32x16_t (&sacc)[2], RowMax &rm, f32x16_t (&acc_o)[DBLK],
-                           float l_run, uint32_t (&pk)[2][8]) {
-  float mx = -INFINITY;
+// Probabilities of one tile, sacc = s - m (masked keys -inf), as bf16 pairs
+// into pk; returns the lane's partial sum of the rounded values the PV
+// product uses (v_dot2c_f32_bf16 with (1, 1)).
+MIA_DEV float exp_tile(const f32x16_t (&sacc)[2], uint32_t (&pk)[2][8]) {
+  typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+  const bf16x2_t ones = {(__bf16)1.0f, (__bf16)1.0f};
+  float psum = 0.f;
 #pragma unroll
   for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-    for (int e = 0; e < 16; ++e) mx = fmaxf(mx, sacc[kb][e]);
-  {  // the other k-group of the row: lanes l and l ^ 32 through one lane swap
-    const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx),
-                                                     false, false);
-    mx = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
-  }
-  const bool bump = rm.set ? (mx > 8.0f) : (mx > -INFINITY);
-  if (__builtin_amdgcn_ballot_w64(bump)) {
+    for (int e = 0; e < 16; e += 2) {
+      const float p0 = __builtin_amdgcn_exp2f(sacc[kb][e]);
+      const float p1 = __builtin_amdgcn_exp2f(sacc[kb][e + 1]);
+      pk[kb][e >> 1] = pack2_bf16(p0, p1);
+      psum = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, pk[kb][e >> 1]), ones,
+                                             psum, false);
+    }
+  return psum;
+}
+
+// max over the two lanes l and l ^ 32 of a row (its two key groups)
+MIA_DEV float row_max2(float x) {
+  const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x),
+                                                   false, false);
+  return fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+}
+
+// One tile of the online softmax over sacc = s - m (masked keys -inf) of
+// the lane's row: probabilities as bf16 pairs into pk, acc_o rescaled when
+// the maximum moves, returns the updated partial sum of the lane.
+// The running maximum moves lazily: to the tile's maximum on the row's first
+// visible key and whenever one of the row's two half sums of the tile passes
+// 2^8, so probabilities stay at or below 2^8 and the accumulators are
+// rescaled only on such tiles.  The test reads the sums, which are there
+// anyway, so a tile computes no maximum (16 v_max3, a lane swap and a wait
+// for all 32 scores before the first exponential): a tile that fails it is
+// recomputed from its scores.
+template <int DBLK>
+MIA_DEV float softmax_tile(f32x16_t (&sacc)[2], RowMax &rm, f32x16_t (&acc_o)[DBLK],
+                           float l_run, uint32_t (&pk)[2][8]) {
+  auto tile_max = [&]() {
+    float mx = -INFINITY;
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) mx = fmaxf(mx, sacc[kb][e]);
+    return row_max2(mx);
+  };
+  // moves the maximum of the rows with `bump` up by mx
+  auto rescale = [&](bool bump, float mx) {
     const float delta = bump ? mx : 0.f;
     // before the first visible key acc_o and l_run are 0: no rescale
     const float alpha = rm.set ? __builtin_amdgcn_exp2f(-delta) : 1.0f;
@@ -507,21 +534,44 @@ MIA_DEV float softmax_tile(f32x16_t (&sacc)[2], RowMax &rm, f32x16_t (&acc_o)[DB
       for (int e = 0; e < 16; ++e) sacc[kb][e] -= delta;
 #pragma unroll
     for (int e = 0; e < 16; ++e) rm.negm[e] = -rm.m;
+  };
+  // both tests depend on the row alone, not on the wave's other rows
+  if (__builtin_expect(__builtin_amdgcn_ballot_w64(!rm.set) != 0, 0)) {
+    const float mx = tile_max();
+    rescale(!rm.set && mx > -INFINITY, mx);
   }
-  typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-  const bf16x2_t ones = {(__bf16)1.0f, (__bf16)1.0f};
-  float psum = 0.f;
-#pragma unroll
-  for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-    for (int e = 0; e < 16; e += 2) {
-      const float p0 = __builtin_amdgcn_exp2f(sacc[kb][e]);
-      const float p1 = __builtin_amdgcn_exp2f(sacc[kb][e + 1]);
-      pk[kb][e >> 1] = pack2_bf16(p0, p1);
-      psum = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, pk[kb][e >> 1]), ones,
-                                             psum, false);
-    }
+  float psum = exp_tile(sacc, pk);
+  if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(psum <= 256.0f)) != 0, 0)) {
+    const float mx = tile_max();
+    rescale(!(row_max2(psum) <= 256.0f), mx);
+    psum = exp_tile(sacc, pk);
+  }
   return l_run + psum;
+}
+
+// Masks the scores of the tile at kt (lane value e of block kb: key kt +
+// kb*32 + (e/4)*8 + half*4 + e%4) outside the row's keys [r_lo, r_hi), each
+// bound only on tiles that some row of the workgroup cuts there ([full_lo,
+// full_hi): the keys every row sees) and relative to the lane's first key,
+// so that the key numbers are immediates.
+MIA_DEV void mask_tile(f32x16_t (&sacc)[2], int kt, int half, int r_lo, int r_hi, int full_lo,
+                       int full_hi) {
+  if (kt + kKT > full_hi) {
+    const int t = r_hi - kt - half * 4;
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+        sacc[kb][e] = kb * 32 + (e >> 2) * 8 + (e & 3) < t ? sacc[kb][e] : -INFINITY;
+  }
+  if (kt < full_lo) {
+    const int t = r_lo - kt - half * 4;
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+        sacc[kb][e] = kb * 32 + (e >> 2) * 8 + (e & 3) >= t ? sacc[kb][e] : -INFINITY;
+  }
 }
 
 // PK: the K cache is in the packed FP8 layout (FP8 only).
@@ -693,6 +743,7 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillKParams p) {
   };
 
   RowMax rm;
+  rm.set = !row_ok;  // rows that are not computed (zero query) never move the maximum
   float l_run = 0.f;        // per lane partial sum
   f32x16_t acc_o[DBLK];
 #pragma unroll
@@ -731,18 +782,7 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillKParams p) {
                                                            0, 0, 0);
       }
     }
-    // lane value e of block kb: key kt + kb*32 + (e/4)*8 + half*4 + e%4
-    const bool full = (kt + kKT <= full_hi) && (kt >= full_lo);
-    if (!full) {
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int key = kt + kb * 32 + (e >> 2) * 8 + half * 4 + (e & 3);
-          const bool ok = row_ok && key < r_hi && key >= r_lo;
-          sacc[kb][e] = ok ? sacc[kb][e] : -INFINITY;
-        }
-    }
+    mask_tile(sacc, kt, half, r_lo, r_hi, full_lo, full_hi);
     // ---- online softmax (log2 domain)
     uint32_t pk[2][8];  // P^T as bf16 pairs, [block][dword]
     l_run = softmax_tile<DBLK>(sacc, rm, acc_o, l_run, pk);
@@ -772,7 +812,7 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillKParams p) {
 }
 
 // ---------------------------------------------------------------------------
-// bf16 cache, head_dim 128: K/V tiles streamed straight into LDS
+// K/V tiles streamed straight into LDS: head_dim 128, and 64 with bf16 caches
 // ---------------------------------------------------------------------------
 // Same products and softmax as prefill_kernel, with 8 waves (256 GQA-packed
 // rows) per workgroup and the 64-key K and V tiles travelling HBM -> LDS
@@ -781,8 +821,10 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillKParams p) {
 // barrier per tile.  The blocks of the workgroup's key range are staged in
 // LDS once, so no global load sits between two tiles' copies.
 // A DMA instruction writes 64 lanes x 16 B contiguously, i.e. 4 rows of
-// 256 B; each lane picks which 16-byte chunk of its row it fetches, which
-// stores the rows XOR-swizzled:
+// 256 B (d = 64: 8 rows of 128 B); each lane picks which 16-byte chunk of its
+// row it fetches, which stores the rows XOR-swizzled (d = 128; d = 64 rows
+// span half the banks, so a row pair shares one swizzle value: s ^ ((r >> 1)
+// & 7) for K, s ^ ((r & 2) << 1) for V):
 //   K: LDS chunk s of row r holds chunk s ^ (r & 15)  -> the 32 lanes that
 //      read one chunk column of 32 rows hit 16 distinct chunk positions;
 //   V: LDS chunk s of row r holds chunk s ^ ((r & 3) << 2) -> conflict-free
@@ -800,8 +842,13 @@ constexpr int kDmaWaves = 8;
 constexpr int kDmaStages = 3;
 constexpr int dma_rows(int waves) { return waves * kRowsW; }
 constexpr int dma_ids(int waves) { return waves == 8 ? 4096 : 2048; }  // block ids in LDS
-constexpr int kDmaRows = dma_rows(kDmaWaves);
+
 constexpr int kDmaIds = dma_ids(kDmaWaves);
+// LDS chunk of row chunk c: c ^ swz(row) (see above).
+template <int D>
+MIA_DEV constexpr int k_swz(int row) { return D == 128 ? row & 15 : (row >> 1) & 7; }
+template <int D>
+MIA_DEV constexpr int v_swz(int row) { return D == 128 ? (row & 3) << 2 : (row & 2) << 1; }
 // s_waitcnt immediate: vmcnt(n), expcnt and lgkmcnt not waited on
 constexpr int waitcnt_vm(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
 static_assert(waitcnt_vm(4) == 0xF74 && waitcnt_vm(0) == 0xF70, "vmcnt encoding");
@@ -813,11 +860,23 @@ static_assert(waitcnt_vm(4) == 0xF74 && waitcnt_vm(0) == 0xF70, "vmcnt encoding"
 // of V per thread, x 2^-8 as in the register kernel), so the products and
 // softmax are those of the bf16 kernel.  PK: K in the packed layout (a
 // 16-byte chunk holds 8 channels of a token pair, interleaved).
+//
+// d = 64 (bf16): half the MFMA work per score, so the exponentials weigh as
+// much as the products, and a tile's 8 + 8 MFMAs are too few to cover LDS
+// reads that the compiler places just before them; all fragments of a product
+// are read ahead (AHEAD).  2048 tokens, 64 q / 8 kv heads, after 4096 tokens
+// (172 GFLOP): 268 us register-staged, 201 us with this ring, 196 us with the
+// row sums as the rescale test, 185-189 us reading ahead; the 128-token window
+// layer 25.5 -> 21.2 us.  Two such workgroups per CU (128 VGPRs) and 4-wave
+// workgroups at three per CU measured 202-209 us: the SIMDs run at the power
+// limit (the clock falls from 2.3 to 1.6 GHz as products and exponentials
+// overlap), so more waves do not help.  Reading ahead at d = 128 costs 1-5 %.
 template <int D, int WAVES, int STAGES, bool FP8, bool PK>
-__global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void prefill_dma_kernel(PrefillKParams p) {
-  static_assert(D == 128, "256-byte rows");
+__global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void prefill_dma_kernel(
+    PrefillKParams p) {
+  static_assert(D == 128 || D == 64, "256- or 128-byte rows");
   static_assert((WAVES == 8 || WAVES == 4) && (STAGES == 2 || STAGES == 3), "ring shape");
-  static_assert(!FP8 || (WAVES == 8 && STAGES == 3), "FP8 ring: one chunk per thread");
+  static_assert(!FP8 || (D == 128 && WAVES == 8 && STAGES == 3), "FP8 ring: one chunk per thread");
   static_assert(FP8 || !PK, "packed K is an FP8 layout");
   constexpr int kDmaWaves = WAVES;
   constexpr int kDmaRows = dma_rows(WAVES);
@@ -826,7 +885,10 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void prefill_dma_kernel(Pref
   constexpr int DBLK = D / 32;
   constexpr int ROWB = D * 2;          // bytes per K/V row
   constexpr int TILEB = kKT * ROWB;    // bytes per K (or V) tile
-  constexpr int NJ = 16 / kDmaWaves;   // DMA instructions per thread per tile (K and V each)
+  constexpr int NJ = TILEB / 1024 / kDmaWaves;  // DMA instructions per thread per tile (K, V each)
+  constexpr int CH = ROWB / 16;        // 16-byte chunks per row
+  constexpr int RPI = 64 / CH;         // rows per DMA instruction
+  constexpr bool AHEAD = D == 64;      // LDS operands read ahead of the products
   constexpr int EB = FP8 ? 1 : 2;      // cache bytes per element
   constexpr int TILE8 = kKT * D;       // bytes per FP8 K (or V) tile
   constexpr int NJ8 = 8 / kDmaWaves;   // FP8 DMA instructions per thread per tile
@@ -835,12 +897,14 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void prefill_dma_kernel(Pref
   typedef __attribute__((address_space(3))) uint8_t lds_u8_t;
 
   // each block of the workgroup's key range (K and V share the block and
-  // token strides on this path): bf16, its byte offset; FP8, its block id
-  // (clamped into the pool), the copies forming the offset (measured: bf16
+  // token strides on this path): bf16 at d = 128, its byte offset; else its
+  // block id (clamped into the pool), the copies forming the offset
+  // (measured at d = 128: bf16
   // 69.3 -> 69.9 us with ids on the 4 x 512 sub-batch and 236.7 -> 237.7 us
   // on the mixed batch's compact launch, FP8 71.3 -> 70.0 us on the
   // 2048-token chunk)
-  typedef std::conditional_t<FP8, int32_t, int64_t> blk_t;
+  constexpr bool IDS = FP8 || D == 64;  // staged as block ids
+  typedef std::conditional_t<IDS, int32_t, int64_t> blk_t;
   __shared__ __attribute__((aligned(16))) blk_t ids_lds[kDmaIds];
   // bf16: [stage][K, V] tiles of the ring; FP8: [buffer][K, V] bf16 tiles
   // the products read, the FP8 ring in kv8_lds
@@ -907,12 +971,12 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void prefill_dma_kernel(Pref
   const int32_t bt0 = tid < n_blk ? p.bt[bt_row + (int64_t)(b_lo + tid) * p.bt_j] : 0;
   auto blk_id = [&](int32_t v) -> blk_t {
     v = v < 0 ? 0 : (v >= p.nb ? p.nb - 1 : v);
-    if constexpr (FP8) return v;
+    if constexpr (IDS) return v;
     else return (int64_t)v * p.kc_blk * EB;
   };
   // byte offset of staged block bi (wave-uniform)
   auto blk_off = [&](int bi) -> int64_t {
-    if constexpr (FP8) {
+    if constexpr (IDS) {
       return (int64_t)readfirstlane(ids_lds[bi]) * p.kc_blk * EB;
     } else {
       const int64_t o = ids_lds[bi];
@@ -948,25 +1012,26 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void prefill_dma_kernel(Pref
   };
   __syncthreads();
 
-  // ---- DMA: instruction j of wave w covers rows 4q .. 4q+3, q = 8j + w;
-  // lane -> row 4q + lane/16, LDS chunk lane % 16.  block_size % 16 == 0,
-  // so the 4 rows of an instruction share a block (a wave-uniform id).
-  // The offset of key kt + row inside its block is (kt % bs) + (row % bs)
-  // (kt % 64 == 0 and either bs divides 64 or 64 divides bs).
-  const int dma_r = lane >> 4;
-  const int dma_s = lane & 15;
+  // ---- DMA: instruction j of wave w covers rows RPI q .. RPI q + RPI - 1,
+  // q = WAVES j + w; lane -> row RPI q + lane / CH, LDS chunk lane % CH.
+  // block_size % 16 == 0, so the 4 (d = 64: 8) rows of an instruction share a
+  // block (a wave-uniform id).  The offset of key kt + row inside its block
+  // is (kt % bs) + (row % bs) (kt % 64 == 0 and either bs divides 64 or 64
+  // divides bs).
+  const int dma_r = lane / CH;
+  const int dma_s = lane % CH;
   const uint8_t *k_head = p.k_cache + (int64_t)h * p.kc_h * 2;
   const uint8_t *v_head = p.v_cache + (int64_t)h * p.vc_h * 2;
   int32_t k_lane[NJ], v_lane[NJ];  // bytes inside a block: < block_size * 256
   int jblk[NJ];  // block of DMA j relative to the tile's first block (wave-uniform)
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
-    const int row = 4 * (kDmaWaves * j + wave) + dma_r;
+    const int row = RPI * (kDmaWaves * j + wave) + dma_r;
     const int roff = row % p.bs;
-    k_lane[j] = roff * (int)p.kc_t * 2 + ((dma_s ^ (row & 15)) << 4);
-    v_lane[j] = roff * (int)p.kc_t * 2 + ((dma_s ^ ((row & 3) << 2)) << 4);
+    k_lane[j] = roff * (int)p.kc_t * 2 + ((dma_s ^ k_swz<D>(row)) << 4);
+    v_lane[j] = roff * (int)p.kc_t * 2 + ((dma_s ^ v_swz<D>(row)) << 4);
     // a 64-key tile starts a block (bs <= 64) or lies inside one (bs > 64)
-    jblk[j] = p.bs <= kKT ? (4 * (kDmaWaves * j + wave)) / p.bs : 0;
+    jblk[j] = p.bs <= kKT ? (RPI * (kDmaWaves * j + wave)) / p.bs : 0;
   }
   // One 16-byte-per-lane copy HBM -> LDS (global_load_lds_dwordx4): lane
   // data lands at lds_dst + 16 * lane.  Issued through inline assembly so
@@ -1000,6 +1065,7 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void prefill_dma_kernel(Pref
   };
 
   RowMax rm;
+  rm.set = !row_ok;  // rows that are not computed (zero query) never move the maximum
   float l_run = 0.f;
   f32x16_t acc_o[DBLK];
 #pragma unroll
@@ -1014,34 +1080,63 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void prefill_dma_kernel(Pref
 
   auto compute_tile = [&](int kt, const lds_u8_t *kb_lds, const lds_u8_t *vb_lds, auto &&after_qk) {
     // ---- S^T = K . Q^T - m (log2 units)
-    f32x16_t sacc[2];
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb) {
+    auto read_k = [&](int kb, int ks) {
       const int row = kb * 32 + rl;
+      const int c = ks * 2 + half;
+      return *(const __attribute__((address_space(3))) u32x4_t *)(kb_lds + row * ROWB +
+                                                                  ((c ^ k_swz<D>(row)) << 4));
+    };
+    f32x16_t sacc[2];
+    if constexpr (AHEAD) {
+      // every K fragment is read before the first product: left to itself
+      // the compiler reads each one just before its MFMA and, with 4 steps
+      // per chain, waits out the LDS latency most times
+      u32x4_t kf[2][KSTEPS];
 #pragma unroll
-      for (int ks = 0; ks < KSTEPS; ++ks) {
-        const int c = ks * 2 + half;
-        const u32x4_t a =
-            *(const __attribute__((address_space(3))) u32x4_t *)(kb_lds + row * ROWB +
-                                                                  ((c ^ (row & 15)) << 4));
-        sacc[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a),
-                                                           qf[ks], ks == 0 ? rm.negm : sacc[kb],
-                                                           0, 0, 0);
-      }
-    }
-    // the copies of a later tile issue while these MFMAs execute
-    after_qk();
-    // lane value e of block kb: key kt + kb*32 + (e/4)*8 + half*4 + e%4
-    const bool full = (kt + kKT <= full_hi) && (kt >= full_lo);
-    if (!full) {
+      for (int ks = 0; ks < KSTEPS; ++ks)
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) kf[kb][ks] = read_k(kb, ks);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int ks = 0; ks < KSTEPS; ++ks)
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+          sacc[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              __builtin_bit_cast(bf16x8_t, kf[kb][ks]), qf[ks], ks == 0 ? rm.negm : sacc[kb], 0,
+              0, 0);
+    } else {
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int key = kt + kb * 32 + (e >> 2) * 8 + half * 4 + (e & 3);
-          const bool ok = row_ok && key < r_hi && key >= r_lo;
-          sacc[kb][e] = ok ? sacc[kb][e] : -INFINITY;
-        }
+        for (int ks = 0; ks < KSTEPS; ++ks)
+          sacc[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              __builtin_bit_cast(bf16x8_t, read_k(kb, ks)), qf[ks],
+              ks == 0 ? rm.negm : sacc[kb], 0, 0, 0);
+    }
+    // the copies of a later tile issue while these MFMAs execute
+    after_qk();
+    mask_tile(sacc, kt, half, r_lo, r_hi, full_lo, full_hi);
+    // V^T fragment of key step ks2 and column block db
+    auto read_v = [&](int ks2, int db) {
+      s16x4_t t2[2];
+#pragma unroll
+      for (int rr = 0; rr < 2; ++rr) {
+        const int row = ks2 * 16 + rr * 8 + tr_row;
+        const int d = db * 32 + tr_col;
+        const int c = d >> 3;
+        const int off = row * ROWB + ((c ^ v_swz<D>(row)) << 4) + ((d & 7) << 1);
+        t2[rr] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t *)(vb_lds + off));
+      }
+      return u32x4_t{__builtin_bit_cast(u32x2_t, t2[0])[0], __builtin_bit_cast(u32x2_t, t2[0])[1],
+                     __builtin_bit_cast(u32x2_t, t2[1])[0], __builtin_bit_cast(u32x2_t, t2[1])[1]};
+    };
+    u32x4_t vf[AHEAD ? 4 : 1][DBLK];
+    if constexpr (AHEAD) {  // the softmax covers the reads of V^T
+#pragma unroll
+      for (int ks2 = 0; ks2 < 4; ++ks2)
+#pragma unroll
+        for (int db = 0; db < DBLK; ++db) vf[ks2][db] = read_v(ks2, db);
+      __builtin_amdgcn_sched_barrier(0);
     }
     uint32_t pk[2][8];
     l_run = softmax_tile<DBLK>(sacc, rm, acc_o, l_run, pk);
@@ -1055,21 +1150,9 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void prefill_dma_kernel(Pref
       const bf16x8_t bop = __builtin_bit_cast(bf16x8_t, bw);
 #pragma unroll
       for (int db = 0; db < DBLK; ++db) {
-        s16x4_t t2[2];
-#pragma unroll
-        for (int rr = 0; rr < 2; ++rr) {
-          const int row = ks2 * 16 + rr * 8 + tr_row;
-          const int d = db * 32 + tr_col;
-          const int c = d >> 3;
-          const int off = row * ROWB + ((c ^ ((row & 3) << 2)) << 4) + ((d & 7) << 1);
-          t2[rr] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t *)(vb_lds + off));
-        }
-        const u32x4_t aw = {__builtin_bit_cast(u32x2_t, t2[0])[0],
-                            __builtin_bit_cast(u32x2_t, t2[0])[1],
-                            __builtin_bit_cast(u32x2_t, t2[1])[0],
-                            __builtin_bit_cast(u32x2_t, t2[1])[1]};
-        acc_o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, aw),
-                                                            bop, acc_o[db], 0, 0, 0);
+        if constexpr (!AHEAD) vf[0][db] = read_v(ks2, db);
+        acc_o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            __builtin_bit_cast(bf16x8_t, vf[AHEAD ? ks2 : 0][db]), bop, acc_o[db], 0, 0, 0);
       }
     }
   };
@@ -1241,7 +1324,7 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void prefill_dma_kernel(Pref
 #pragma unroll
     for (int e4 = 0; e4 < 4; ++e4) {
       const int c = db * 4 + e4;  // 16-byte chunk of the row; half picks its 8 bytes
-      *(__attribute__((address_space(3))) u32x2_t *)(ob + rl * ROWB + ((c ^ (rl & 15)) << 4) +
+      *(__attribute__((address_space(3))) u32x2_t *)(ob + rl * ROWB + ((c ^ (rl & (CH - 1))) << 4) +
                                                      half * 8) =
           u32x2_t{pack2_bf16(acc_o[db][e4 * 4] * rscale, acc_o[db][e4 * 4 + 1] * rscale),
                   pack2_bf16(acc_o[db][e4 * 4 + 2] * rscale, acc_o[db][e4 * 4 + 3] * rscale)};
@@ -1252,13 +1335,12 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void prefill_dma_kernel(Pref
     *reinterpret_cast<float2 *>(w + 2 * D) = make_float2(m_fin, l_run);
   }
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wave's rows are in LDS
-  constexpr int CH = ROWB / 16;  // 16-byte chunks per row
   const bool out16 = (((uintptr_t)p.out | (uint32_t)(p.os_t | p.os_h) * 2u) & 15u) == 0;
 #pragma unroll
   for (int i = 0; i < kRowsW * CH / 64; ++i) {
     const int rl2 = i * (64 / CH) + lane / CH, ch = lane % CH;
     const u32x4_t v = *(const __attribute__((address_space(3))) u32x4_t *)(
-        ob + rl2 * ROWB + ((ch ^ (rl2 & 15)) << 4));
+        ob + rl2 * ROWB + ((ch ^ (rl2 & (CH - 1))) << 4));
     const int r2 = row0 + wave * kRowsW + rl2;
     const int pos2 = r2 / G;
     if (r2 >= rows_total || q_begin + pos2 >= p.num_tokens) continue;
@@ -1383,7 +1465,10 @@ bool use_dma_kernel(const mia_prefill_args &a) {
   // the copies address K and V with one block offset and one token stride
   // (packed K: the stride of the even token of a pair)
   const int64_t k_tok = a.k_packed ? a.k_cache_stride[2] / 2 : a.k_cache_stride[2];
-  return a.head_dim == 128 && dtype_ok && a.block_size % 16 == 0 &&
+  // d = 64: bf16 caches.  Compact launches and FP8 caches of that head dim
+  // keep the register-staged kernel.
+  const bool dim_ok = a.head_dim == 128 || (a.cache_dtype == MIA_DTYPE_BF16 && !a.compact_kernel);
+  return dim_ok && dtype_ok && a.block_size % 16 == 0 &&
          k_tok == a.v_cache_stride[2] &&
          (64 % a.block_size == 0 || a.block_size % 64 == 0) && a.blocks_per_seq <= kDmaIds &&
          a.k_cache_stride[0] == a.v_cache_stride[0];
@@ -1505,7 +1590,10 @@ int launch_paged_prefill(const mia_prefill_args &a, const PrefillPlan &pl, hipSt
   kp.rank_items = a.num_seqs > 1 ? 1 : 0;
   const dim3 grid((unsigned)((pl.rows_max + pl.rows_wg - 1) / pl.rows_wg),
                   (unsigned)a.num_kv_heads, (unsigned)(pl.nsplit * a.num_seqs));
-  if (pl.dma && pl.dma_waves == 4) {
+  if (pl.dma && a.head_dim == 64) {
+    hipLaunchKernelGGL((prefill_dma_kernel<64, kDmaWaves, kDmaStages, false, false>), grid,
+                       dim3(kDmaWaves * 64), 0, s, kp);
+  } else if (pl.dma && pl.dma_waves == 4) {
     hipLaunchKernelGGL((prefill_dma_kernel<128, 4, 2, false, false>), grid, dim3(4 * 64), 0, s,
                        kp);
   } else if (pl.dma) {
