@@ -397,3 +397,53 @@ def test_copy_ring_tile_edges_and_rising_scores(gpu, d, bs, new, prior, window, 
                          None if sink is None else sink.cpu())
     err = (out.float().cpu().double() - f).abs().max().item()
     assert err <= TOL_BF16 + 4 * 4.5e-3, err
+
+
+EVEN_CASES = [
+    # q heads, kv heads, d, bs, new, prior, table tokens, window, sink, fp8
+    (8, 2, 128, 32, 1, 4096, 0, 0, False, False),      # one row, 4-wave workgroups
+    (32, 8, 128, 16, 200, 5000 // 16 * 16, 0, 0, True, False),   # 8-wave, 8 chunks
+    (32, 8, 128, 32, 65, 640, 16384, 0, True, False),  # table far wider than the sequence
+    (8, 1, 64, 64, 33, 9600, 0, 0, True, False),       # 32 chunks, one kv head
+    (64, 8, 64, 32, 1100, 4096, 0, 0, True, False),    # whole rounds of uncut row tiles
+    (32, 8, 64, 16, 130, 6000 // 16 * 16, 0, 1500, False, False),  # window cut across chunks
+    (12, 2, 128, 64, 100, 4096, 0, 0, False, True),    # FP8 ring
+    (12, 2, 64, 64, 100, 4096, 0, 0, True, True),      # FP8, register-staged kernel
+]
+
+
+@pytest.mark.parametrize("case", range(len(EVEN_CASES)))
+def test_single_sequence_even_split(gpu, case):
+    """One sequence whose row tiles are cut evenly on the device: equal to the
+    uncut launch within two bf16 steps (each chunk keeps its own running
+    maximum; partials are fp32), and within tolerance of float64 math."""
+    Hq, Hkv, d, bs, new, prior, wide, win, use_sink, fp8 = EVEN_CASES[case]
+    cfg = W.PrefillConfig("e", 1, Hq, Hkv, d, bs, new, prior, prior, fp8=fp8, seed=170 + case)
+    b = W.make_prefill_batch(cfg, gpu)
+    kw = {}
+    if fp8:
+        kw = dict(k_dequant=b.k_dequant, v_dequant=b.v_dequant)
+        K.kv_write(b.k_new, b.v_new, b.slots, b.k_cache, b.v_cache, quant_mode=2,
+                   k_scale=b.k_quant, v_scale=b.v_quant, scale_per_head=True)
+    else:
+        K.kv_write(b.k_new, b.v_new, b.slots, b.k_cache, b.v_cache)
+    table = b.block_table
+    if wide:
+        table = torch.full((1, wide // bs), -1, dtype=torch.int32, device=gpu)
+        table[:, :b.block_table.shape[1]] = b.block_table
+    sink = torch.randn(Hq, generator=torch.Generator().manual_seed(case)).to(gpu) if use_sink else None
+    run = lambda split: K.paged_prefill(b.q, b.cu_seqlens, b.prior, new, b.k_cache, b.v_cache, table,
+                                        scale=d ** -0.5, sliding_window=win, sink=sink,
+                                        split_tokens=split, **kw)
+    got, base = run(0), run(1 << 20)
+    assert (got.float() - base.float()).abs().max().item() <= 1.6e-2
+    n, first = prior + new, max(0, new - 40)  # float64 on the last rows
+    kc, vc = b.k_cache.cpu(), b.v_cache.cpu()
+    if fp8:
+        kc = kc.float() * b.k_dequant.cpu().view(1, -1, 1, 1)
+        vc = vc.float() * b.v_dequant.cpu().view(1, -1, 1, 1)
+    ks, vs = (_seq_kv(c, b.block_table[0].cpu(), n, Hkv) for c in (kc, vc))
+    f = OSg.fp32_prefill(b.q[first:].cpu(), ks, vs, prior + first, d ** -0.5, win,
+                         None if sink is None else sink.cpu())
+    err = (got[first:].float().cpu().double() - f).abs().max().item()
+    assert err <= (TOL_FP8 if fp8 else TOL_BF16), err

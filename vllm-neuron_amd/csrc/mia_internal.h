@@ -60,12 +60,16 @@ int launch_decode_scatter(const mia_decode_args &a, hipStream_t s);
 
 // Paged prefill: split-K plan shared by the workspace query and the launch.
 struct PrefillPlan {
-  bool dma;          // bf16 / head_dim 128 kernel with the LDS copy ring
-  int dma_waves;     // its waves per workgroup (8, or 4 for compact launches)
+  bool dma;          // kernel with the LDS copy ring
+  int dma_waves;     // its waves per workgroup (8, or 4 for compact launches
+                     // and short single sequences)
   int rows_wg;       // query rows per workgroup
   int rows_max;      // max_seqlen_q * G
   int nsplit;        // key chunks per row tile at most (1: no split)
   int ksplit;        // keys per chunk (0: chosen on the device)
+  bool even;         // one sequence, cut evenly on the device (fp32 partials)
+  int whole;         // even: row tiles left uncut
+  int row_tiles;     // even: row tiles of the launch
   int slots;         // workgroups resident on the device at once
   size_t ws_bytes;   // workspace bytes (0 without split)
 };

@@ -49,7 +49,13 @@ constexpr int kVPad = 8;      // bf16 padding per V^T row in LDS
 // a split partial row: o[D] as bf16, then m and l (fp32) and 8 bytes of
 // padding (rows stay 16-byte aligned)
 constexpr int part_bytes(int D) { return 2 * D + 16; }
-constexpr int kMaxChunks = 8; // key chunks of a split row tile at most
+constexpr int kMaxChunks = 8; // chunks of ksplit keys of a split row tile at most
+// Even split of one sequence: chunks per row tile at most, key tiles per
+// chunk at least, and its partial row: o[D], m, l as fp32 and 8 bytes of
+// padding.
+constexpr int kMaxEven = 32;
+constexpr int kMinEvenTiles = 4;
+constexpr int part32_bytes(int D) { return 4 * D + 16; }
 
 struct PrefillKParams {
   const uint16_t *q;
@@ -79,6 +85,10 @@ struct PrefillKParams {
   int nsplit;     // chunks per row tile at most (grid z = nsplit * num_seqs)
   int num_seqs;
   int ksplit;     // keys per chunk (multiple of the 64-key tile)
+  int even;       // one sequence: each row tile's key tiles cut into up to
+                  // nsplit equal chunks, partials in fp32
+  int whole;      // even: row tiles (of the grid's last rows) left uncut
+  int row_tiles;  // even: row tiles of the grid
   int slots;      // workgroups resident on the device at once
   int rows_wg;    // query rows per workgroup of the attention kernel
   int rows_max;   // max_seqlen_q * G
@@ -180,8 +190,30 @@ MIA_DEV KeyRange wg_key_range(const PrefillKParams &p, int seq, int prior, int S
   k.any = k.kmax > k.kmin;
   k.kt0 = (k.kmin / kKT) * kKT;
   k.kt_last = k.kmax > k.kt0 ? ((k.kmax - 1) / kKT) * kKT : k.kt0;
-  k.n_sp = (k.any && p.nsplit > 1) ? k.kt_last / ksplit - k.kt0 / ksplit + 1 : 1;
+  if (p.even)
+    k.n_sp = k.any && row0 / p.rows_wg < p.row_tiles - p.whole
+                 ? min(max(((k.kt_last - k.kt0) / kKT + 1) / kMinEvenTiles, 1), p.nsplit)
+                 : 1;
+  else
+    k.n_sp = (k.any && p.nsplit > 1) ? k.kt_last / ksplit - k.kt0 / ksplit + 1 : 1;
   return k;
+}
+
+// First and last tile of chunk sp of the key range.
+MIA_DEV void chunk_tiles(const PrefillKParams &p, const KeyRange &k, int ksplit, int sp, int &kt0,
+                         int &kt_last) {
+  kt0 = k.kt0;
+  kt_last = k.kt_last;
+  if (k.n_sp <= 1) return;
+  if (p.even) {
+    const int n = (k.kt_last - k.kt0) / kKT + 1;
+    kt0 = k.kt0 + n * sp / k.n_sp * kKT;
+    kt_last = k.kt0 + (n * (sp + 1) / k.n_sp - 1) * kKT;
+  } else {
+    const int c = k.kt0 / ksplit + sp;
+    kt0 = max(k.kt0, c * ksplit);
+    kt_last = min(k.kt_last, c * ksplit + ksplit - kKT);
+  }
 }
 
 // Workgroups are dispatched to the 8 XCDs round-robin by linear id, and each
@@ -191,7 +223,10 @@ MIA_DEV KeyRange wg_key_range(const PrefillKParams &p, int seq, int prior, int S
 // consecutive XCDs (group g on XCD g % 8), groups of higher chunk index last
 // within each XCD.  When the group count is not a multiple of 8 the launch
 // order is kept.
-MIA_DEV uint3 xcd_tile() {
+// One sequence with an even split: a group's items are its uncut row tiles,
+// then the chunks of the others, tile by tile (grid.x = whole + (row tiles -
+// whole) * nsplit).
+MIA_DEV uint3 xcd_tile(const PrefillKParams &p) {
   constexpr uint32_t X = 8;
   const uint32_t R = gridDim.x;                 // row tiles per group
   const uint32_t groups = gridDim.y * gridDim.z;
@@ -201,6 +236,14 @@ MIA_DEV uint3 xcd_tile() {
     const uint32_t x = L % X, k = L / X;         // k-th workgroup of XCD x
     rt = k % R;
     g = (k / R) * X + x;
+  }
+  if (p.even) {
+    const uint32_t W = (uint32_t)p.whole, n = (uint32_t)p.nsplit;
+    uint3 t;
+    t.x = (uint32_t)p.row_tiles - 1 - (rt < W ? rt : W + (rt - W) / n);
+    t.y = g % gridDim.y;
+    t.z = rt < W ? 0 : (rt - W) % n;
+    return t;
   }
   // heaviest row tile first: under the causal mask the last rows see the
   // most keys, and starting them first shortens the tail (2048-token causal
@@ -246,12 +289,8 @@ MIA_DEV int item_cost(const PrefillKParams &p, int rt, int g, SeqInfo &si) {
   const KeyRange kr = wg_key_range(p, seq, si.prior, S_q, row0, ksplit);
   if (sp >= kr.n_sp) return 0;
   if (!kr.any) return 1;
-  int kt0 = kr.kt0, kt_last = kr.kt_last;
-  if (kr.n_sp > 1) {
-    const int c = kt0 / ksplit + sp;
-    kt0 = max(kt0, c * ksplit);
-    kt_last = min(kt_last, c * ksplit + ksplit - kKT);
-  }
+  int kt0, kt_last;
+  chunk_tiles(p, kr, ksplit, sp, kt0, kt_last);
   return (kt_last - kt0) / kKT + 2;
 }
 
@@ -311,7 +350,7 @@ MIA_DEV uint3 ranked_tile(const PrefillKParams &p, int *scratch, int cap, SeqInf
   const uint32_t mo = (n_x + 4) & ~3u;
   if (!p.rank_items || groups % X != 0 || mo + 4 * n_x > (uint32_t)cap || n_x > kRankMax ||
       n_x > NT) {
-    const uint3 t = xcd_tile();
+    const uint3 t = xcd_tile(p);
     info = load_seq(p, (int)(t.z % (uint32_t)p.num_seqs));
     return t;
   }
@@ -396,11 +435,33 @@ MIA_DEV void store_final(const PrefillKParams &p, const f32x16_t (&acc_o)[D / 32
   }
 }
 
+// This chunk's fp32 partial (o * vscale, m, l) of one row for the merge of an
+// even split: the merged row is rounded to bf16 once, as an unsplit row is.
+// l_run is the row's full sum.
+template <int D>
+MIA_DEV void store_part32(const PrefillKParams &p, const f32x16_t (&acc_o)[D / 32], float m_run,
+                          float l_run, int h, int r, int half, int sp, float vscale) {
+  float *w = reinterpret_cast<float *>(
+      p.ws + (((int64_t)h * p.rows_max + r) * p.nsplit + sp) * (int64_t)part32_bytes(D));
+#pragma unroll
+  for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+    for (int e4 = 0; e4 < 4; ++e4)
+      *reinterpret_cast<float4 *>(w + db * 32 + e4 * 8 + half * 4) =
+          make_float4(acc_o[db][e4 * 4] * vscale, acc_o[db][e4 * 4 + 1] * vscale,
+                      acc_o[db][e4 * 4 + 2] * vscale, acc_o[db][e4 * 4 + 3] * vscale);
+  if (half == 0) *reinterpret_cast<float2 *>(w + D) = make_float2(m_run, l_run);
+}
+
 template <int D>
 MIA_DEV void finish_rows(const PrefillKParams &p, const f32x16_t (&acc_o)[D / 32], float m_run,
                          float l_run, bool row_ok, int seq, int h, int hq, int64_t tok,
                          int r, int half, int n_sp, int sp, float vscale) {
   l_run += __shfl_xor(l_run, 32, 64);
+  if (n_sp > 1 && p.even) {
+    if (row_ok) store_part32<D>(p, acc_o, m_run, l_run, h, r, half, sp, vscale);
+    return;
+  }
   if (n_sp > 1) {
     // split row tile: store this chunk's partial (o * vscale as bf16, m,
     // l) for prefill_combine_kernel; bf16 o halves the partial traffic and
@@ -664,12 +725,8 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillKParams p) {
   const int v_col = (vg >> 2) * 16 + (((vg & 1) << 1) | ((vg >> 1) & 1)) * 4;
 
   if (sp >= kr.n_sp) return;  // no chunk for this workgroup
-  int kt0 = kr.kt0, kt_last = kr.kt_last;
-  if (kr.n_sp > 1) {
-    const int c = kt0 / ksplit + sp;
-    kt0 = max(kt0, c * ksplit);
-    kt_last = min(kt_last, c * ksplit + ksplit - kKT);
-  }
+  int kt0, kt_last;
+  chunk_tiles(p, kr, ksplit, sp, kt0, kt_last);
   // clamp a key into [kt0, kmax) so every load hits an attended block
   auto clampk = [&](int k) { return min(max(k, kt0), max(kmax - 1, kt0)); };
   auto phys_of = [&](int key) {
@@ -951,12 +1008,8 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void prefill_dma_kernel(
   const int full_lo = kr.full_lo;
   const bool any_key = kr.any;
   if (sp >= kr.n_sp) return;  // no chunk for this workgroup
-  int kt0 = kr.kt0, kt_last = kr.kt_last;
-  if (kr.n_sp > 1) {
-    const int c = kt0 / ksplit + sp;
-    kt0 = max(kt0, c * ksplit);
-    kt_last = min(kt_last, c * ksplit + ksplit - kKT);
-  }
+  int kt0, kt_last;
+  chunk_tiles(p, kr, ksplit, sp, kt0, kt_last);
 
   // Q pre-multiplied by the softmax scale (log2 units) and rounded to bf16,
   // so that the MFMA yields scaled scores and the softmax needs no multiply
@@ -1319,6 +1372,42 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void prefill_dma_kernel(
   }
   __syncthreads();
   lds_u8_t *const ob = kv_base + wave * (kRowsW * ROWB);
+  if (split && p.even) {
+    // fp32 partial, half the row's columns at a time: ROWB bytes per row
+    constexpr int DBP = DBLK / 2;
+    float *const part = reinterpret_cast<float *>(p.ws);
+    const int64_t step = (int64_t)p.nsplit * (part32_bytes(D) / 4);
+    const int64_t first = ((int64_t)h * p.rows_max + row0 + wave * kRowsW) * step +
+                          (int64_t)sp * (part32_bytes(D) / 4);
+#pragma unroll
+    for (int pass = 0; pass < 2; ++pass) {
+#pragma unroll
+      for (int db = 0; db < DBP; ++db)
+#pragma unroll
+        for (int e4 = 0; e4 < 4; ++e4) {
+          const int c = db * 8 + e4 * 2 + half;
+          const f32x16_t &a = acc_o[pass * DBP + db];
+          *(__attribute__((address_space(3))) f32x4_t *)(ob + rl * ROWB +
+                                                         ((c ^ (rl & (CH - 1))) << 4)) =
+              f32x4_t{a[e4 * 4] * vscale, a[e4 * 4 + 1] * vscale, a[e4 * 4 + 2] * vscale,
+                      a[e4 * 4 + 3] * vscale};
+        }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wave's rows are in LDS
+#pragma unroll
+      for (int i = 0; i < kRowsW * CH / 64; ++i) {
+        const int rl2 = i * (64 / CH) + lane / CH, ch = lane % CH;
+        const f32x4_t v = *(const __attribute__((address_space(3))) f32x4_t *)(
+            ob + rl2 * ROWB + ((ch ^ (rl2 & (CH - 1))) << 4));
+        const int r2 = row0 + wave * kRowsW + rl2;
+        if (r2 < rows_total && q_begin + r2 / G < p.num_tokens)
+          *reinterpret_cast<f32x4_t *>(part + first + rl2 * step + pass * (D / 2) + ch * 4) = v;
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // read before the next pass writes
+    }
+    if (row_ok && half == 0)
+      *reinterpret_cast<float2 *>(part + first + rl * step + D) = make_float2(m_fin, l_run);
+    return;
+  }
 #pragma unroll
   for (int db = 0; db < DBLK; ++db)
 #pragma unroll
@@ -1442,6 +1531,75 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(PrefillKParams p) 
   }
 }
 
+// Merge of an even split's fp32 partials: D/8 lanes per row (8 floats each), one
+// row step per wave, so that a short launch (few rows, up to 32 chunks) still
+// spreads over the chip; 8 chunks' loads in flight, batches merged online.
+template <int D>
+__global__ __launch_bounds__(256) void prefill_merge32_kernel(PrefillKParams p) {
+  constexpr int LPR = D / 8;
+  constexpr int RPS = 64 / LPR;
+  constexpr int PB = part32_bytes(D);
+  constexpr int kBatch = 8;
+  const int h = blockIdx.y;
+  const int q_begin = p.cu[0];
+  const int S_q = p.cu[1] - q_begin;
+  const int rows_total = S_q * p.G;
+  const int lane = threadIdx.x & 63;
+  const int r = ((int)blockIdx.x * 4 + (int)(threadIdx.x >> 6)) * RPS + lane / LPR;
+  // the rows of a wave lie in one row tile (rows_wg % 8 == 0)
+  const int row0 = (int)blockIdx.x * 4 * RPS;
+  if (row0 >= rows_total) return;
+  const KeyRange kr =
+      wg_key_range(p, 0, p.prior[0], S_q, (row0 / p.rows_wg) * p.rows_wg, split_keys(p));
+  if (kr.n_sp <= 1 || r >= rows_total) return;
+  const int pos_r = r / p.G;
+  const int hq = h * p.G + (r - pos_r * p.G);
+  const int c8 = (lane % LPR) * 8;
+  const uint8_t *w0 = p.ws + ((int64_t)h * p.rows_max + r) * p.nsplit * (int64_t)PB;
+  const float sink2 = p.sink ? p.sink[hq] * kLog2e : -INFINITY;
+  float M = sink2, L = p.sink ? 1.0f : 0.f;  // the sink joins the denominator
+  float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  for (int j0 = 0; j0 < kr.n_sp; j0 += kBatch) {
+    f32x4_t o[kBatch][2];
+    float2 ml[kBatch];
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j) {
+      // past the last chunk: chunk 0 again, with weight 0
+      const uint8_t *w = w0 + (j0 + j < kr.n_sp ? j0 + j : 0) * PB;
+      ml[j] = *reinterpret_cast<const float2 *>(w + 4 * D);
+      o[j][0] = *reinterpret_cast<const f32x4_t *>(w + 4 * c8);
+      o[j][1] = *reinterpret_cast<const f32x4_t *>(w + 4 * c8 + 16);
+    }
+    float Mn = M;
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j)
+      if (j0 + j < kr.n_sp) Mn = fmaxf(Mn, ml[j].x);
+    const float Mu = (Mn == -INFINITY) ? 0.f : Mn;
+    const float f0 = __builtin_amdgcn_exp2f(M - Mu);
+    L *= f0;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[e] *= f0;
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j) {
+      if (j0 + j < kr.n_sp) {
+        const float f = __builtin_amdgcn_exp2f(ml[j].x - Mu);
+        L += ml[j].y * f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[e] += o[j][e >> 2][e & 3] * f;
+      }
+    }
+    M = Mn;
+  }
+  if (q_begin + pos_r >= p.num_tokens) return;
+  const float inv = L > 0.f ? 1.0f / L : 0.f;
+  uint16_t *op = p.out + (int64_t)(q_begin + pos_r) * p.os_t + (int64_t)hq * p.os_h + c8;
+  // two 8-byte stores: the output is only 8-byte aligned
+  *reinterpret_cast<u32x2_t *>(op) =
+      u32x2_t{pack2_bf16(acc[0] * inv, acc[1] * inv), pack2_bf16(acc[2] * inv, acc[3] * inv)};
+  *reinterpret_cast<u32x2_t *>(op + 4) =
+      u32x2_t{pack2_bf16(acc[4] * inv, acc[5] * inv), pack2_bf16(acc[6] * inv, acc[7] * inv)};
+}
+
 }  // namespace
 
 namespace {
@@ -1476,8 +1634,94 @@ bool use_dma_kernel(const mia_prefill_args &a) {
 
 }  // namespace
 
+namespace {
+
+// Launch of one sequence.  The host knows the new tokens and, from the table's
+// width, the most keys a row tile can see; a row tile that sees fewer is cut
+// into fewer chunks by the kernel (kMinEvenTiles).  Uncut, a short chunk after a
+// long context is a few workgroups that each walk the whole context: 200 tokens
+// after 8000 (32 q / 8 kv heads, d = 128) took 208 us on 32 of 256 CUs.
+//
+// Choices: 8-wave workgroups (256 rows, one per CU) with every row tile cut
+// into n chunks, or only the row tiles left over after whole rounds of uncut
+// ones (fewer partials); 4-wave workgroups (128 rows, up to two per CU), cut or
+// not.  Each is estimated (us) as the longest item or the slots' share of all
+// items, whichever is more, a fixed cost per item and the merge's launch and
+// traffic.  Rates measured per 64-key tile: d = 128, 1.6 us for an 8-wave
+// workgroup (FP8 1.85), 1.27 us for a 4-wave one alone on its CU and 2.1 us for
+// two; d = 64, 1.0 / 0.75 / 1.15 us.  Start and epilogue of an item take ~6 us.
+// A plan of ksplit-key chunks already in pl (a long table under few row tiles)
+// keeps its bf16 partials and is taken unless another choice is 5 % better.
+// Measured before and now (us; new tokens after prior ones): 777 / 1536 64 -> 52,
+// 200 / 8000 125 -> 49, 64 / 16000 213 -> 41 (llama-like, d = 128, 32 q / 8 kv);
+// 100 / 4096 51 -> 22, 1200 / 12000 409 -> 299 (d = 64); FP8 300 / 4096 89 -> 58.
+void plan_even(const mia_prefill_args &a, bool half_ok, PrefillPlan &pl) {
+  const int D = a.head_dim;
+  const double t8 = a.cache_dtype != MIA_DTYPE_BF16 ? 1.85 : D == 128 ? 1.6 : 1.0;
+  const double t4 = D == 128 ? 1.27 : 0.75, t4x2 = D == 128 ? 2.1 : 1.15;
+  const double fixed = 6.0;
+  const int cus = device_cus(), Hkv = a.num_kv_heads;
+  const int rows8 = pl.rows_wg;
+  // key tiles that the last row tile sees (T) and a mean one (causal: fewer by
+  // half the new tokens)
+  double keys = (double)a.blocks_per_seq * a.block_size;
+  if (!a.non_causal && a.sliding_window > 0)
+    keys = std::min(keys, a.sliding_window + (double)rows8 * Hkv / a.num_q_heads + kKT - 1);
+  const double drop =
+      a.non_causal || a.sliding_window > 0 ? 0.0 : std::min<double>(a.max_seqlen_q, keys) / kKT;
+  const double T = std::max(1.0, keys / kKT);
+  const int R = (pl.rows_max + rows8 - 1) / rows8, R4 = (pl.rows_max + 127) / 128;
+  auto merge = [&](double rows, int n, int row_bytes) {
+    return n > 1 ? 6.0 + std::min<double>(rows, pl.rows_max) * Hkv * n * row_bytes * 2 / 4.5e6
+                 : 0.0;
+  };
+  // 8-wave workgroups: the last `cut` row tiles in n chunks
+  auto cut8 = [&](int cut, int n, double far, int row_bytes) {
+    const double mean = std::max(1.0, far - drop * cut / R / 2);
+    const double rounds = std::ceil((double)cut * n * Hkv / cus);
+    return std::max(far / n, rounds * mean / n) * t8 + rounds * fixed +
+           merge((double)cut * rows8, n, row_bytes);
+  };
+  double best = pl.nsplit > 1 ? cut8(R, pl.nsplit, T, part_bytes(D)) : 1e30;
+  auto offer = [&](double est, int n, int whole, int waves, int rows) {
+    if (est >= (n > 1 || !pl.even ? 0.95 : 1.0) * best) return;
+    pl.even = true;
+    best = est;
+    pl.nsplit = n;
+    pl.whole = whole;
+    pl.dma_waves = waves;
+    pl.rows_wg = rows;
+  };
+  const int per_head = std::max(1, cus / Hkv);  // row tiles of a head in one round
+  for (int n = 1; n <= kMaxEven; n += n < 4 ? 1 : n < 8 ? 2 : n < 16 ? 4 : 8) {
+    if (n > 1 && T / n < kMinEvenTiles) break;
+    for (const int whole : {0, (R - 1) / per_head * per_head}) {
+      if (whole && n == 1) continue;
+      offer((whole ? whole / per_head * (T * t8 + fixed) : 0.0) +
+                cut8(R - whole, n, T - drop * whole / R, part32_bytes(D)),
+            n, whole, kDmaWaves, rows8);
+    }
+    if (half_ok) {
+      // whole rounds of two per CU, heavy items beside light ones, then the rest
+      const double mean = std::max(1.0, T - drop / 2), len = (T + mean) / 2 / n;
+      const double fill = (double)R4 * n * Hkv / cus;  // workgroups per CU
+      const double full = std::floor(fill / 2), rest = fill - 2 * full;
+      const double t = rest > 0 ? t4 + (t4x2 - t4) * std::max(0.0, rest - 1) : 0.0;
+      offer(std::max(T / n * t4, len * (full * t4x2 + t)) + std::ceil(fill / 2) * fixed +
+                merge((double)pl.rows_max, n, part32_bytes(D)),
+            n, 0, 4, 128);
+    }
+  }
+  if (!pl.even) return;
+  pl.ksplit = 1 << 30;
+  pl.row_tiles = (pl.rows_max + pl.rows_wg - 1) / pl.rows_wg;
+  pl.ws_bytes = pl.nsplit > 1 ? (size_t)Hkv * pl.rows_max * pl.nsplit * part32_bytes(D) : 0;
+}
+
+}  // namespace
+
 PrefillPlan plan_prefill(const mia_prefill_args &a) {
-  PrefillPlan pl;
+  PrefillPlan pl{};
   // compact: workgroups that fit on a CU beside a decode workgroup (the
   // copy ring with 4 waves and 2 stages, 72 KiB of LDS; FP8 caches and
   // shapes the ring does not take use the register-staged kernel)
@@ -1529,6 +1773,9 @@ PrefillPlan plan_prefill(const mia_prefill_args &a) {
     pl.ws_bytes = (size_t)a.num_seqs * a.num_kv_heads * pl.rows_max * pl.nsplit *
                   part_bytes(a.head_dim);
   }
+  if (a.split_tokens <= 0 && a.num_seqs == 1 && !a.compact_kernel && !a.bound_min &&
+      pl.rows_max > 0)
+    plan_even(a, pl.dma && a.cache_dtype == MIA_DTYPE_BF16 && a.blocks_per_seq <= dma_ids(4), pl);
   return pl;
 }
 
@@ -1575,6 +1822,9 @@ int launch_paged_prefill(const mia_prefill_args &a, const PrefillPlan &pl, hipSt
   kp.ws = (uint8_t *)a.workspace;
   kp.nsplit = pl.nsplit;
   kp.ksplit = pl.ksplit;
+  kp.even = pl.even ? 1 : 0;
+  kp.whole = pl.whole;
+  kp.row_tiles = pl.row_tiles;
   kp.slots = pl.slots;
   kp.num_seqs = a.num_seqs;
   kp.rows_wg = pl.rows_wg;
@@ -1588,9 +1838,15 @@ int launch_paged_prefill(const mia_prefill_args &a, const PrefillPlan &pl, hipSt
   kp.q_off = a.q_offset;
   kp.uniform = a.empty_rows_uniform ? 1 : 0;
   kp.rank_items = a.num_seqs > 1 ? 1 : 0;
-  const dim3 grid((unsigned)((pl.rows_max + pl.rows_wg - 1) / pl.rows_wg),
-                  (unsigned)a.num_kv_heads, (unsigned)(pl.nsplit * a.num_seqs));
-  if (pl.dma && a.head_dim == 64) {
+  const dim3 grid = pl.even ? dim3((unsigned)(pl.whole + (pl.row_tiles - pl.whole) * pl.nsplit),
+                                   (unsigned)a.num_kv_heads, 1u)
+                            : dim3((unsigned)((pl.rows_max + pl.rows_wg - 1) / pl.rows_wg),
+                                   (unsigned)a.num_kv_heads,
+                                   (unsigned)(pl.nsplit * a.num_seqs));
+  if (pl.dma && a.head_dim == 64 && pl.dma_waves == 4) {
+    hipLaunchKernelGGL((prefill_dma_kernel<64, 4, kDmaStages, false, false>), grid, dim3(4 * 64),
+                       0, s, kp);
+  } else if (pl.dma && a.head_dim == 64) {
     hipLaunchKernelGGL((prefill_dma_kernel<64, kDmaWaves, kDmaStages, false, false>), grid,
                        dim3(kDmaWaves * 64), 0, s, kp);
   } else if (pl.dma && pl.dma_waves == 4) {
@@ -1617,6 +1873,15 @@ int launch_paged_prefill(const mia_prefill_args &a, const PrefillPlan &pl, hipSt
   }
   int rc = check_hip(hipGetLastError(), "prefill launch");
   if (rc || pl.nsplit <= 1) return rc;
+  if (pl.even) {
+    const int rows = 4 * 64 / (a.head_dim / 8);  // per workgroup
+    const dim3 mgrid((unsigned)((pl.rows_max + rows - 1) / rows), (unsigned)a.num_kv_heads, 1u);
+    if (a.head_dim == 128)
+      hipLaunchKernelGGL((prefill_merge32_kernel<128>), mgrid, dim3(256), 0, s, kp);
+    else
+      hipLaunchKernelGGL((prefill_merge32_kernel<64>), mgrid, dim3(256), 0, s, kp);
+    return check_hip(hipGetLastError(), "prefill merge launch");
+  }
   const dim3 cgrid((unsigned)((pl.rows_max + 63) / 64), (unsigned)a.num_kv_heads,
                    (unsigned)a.num_seqs);
   if (a.head_dim == 128)
