@@ -429,3 +429,35 @@ def test_attention_decode_projection_stages(gpu, fp8):
         gf, rf = got.float().permute(0, 2, 1, 3)[written], r.float().permute(0, 2, 1, 3)[written]
         tol = 0.13 * rf.abs() + 0.05 if fp8 else 2e-2 * rf.abs().clamp_min(1)
         assert ((gf - rf).abs() <= tol).all()
+
+
+@pytest.mark.parametrize("mode", [N.QUANT_NONE, N.QUANT_MUL_BF16, N.QUANT_MUL_F32, N.QUANT_DIV_F32])
+@pytest.mark.parametrize("packed", [False, True])
+def test_epilogue_fp8_codes_of_every_bf16_value(gpu, mode, packed):
+    """Every bf16 bit pattern (infinities, NaN, denormals and both zeros
+    among them) through the epilogue's FP8 write: the bytes of mia_kv_write,
+    which converts in integer arithmetic, and the bf16 row unchanged (NaN
+    stays NaN)."""
+    T, Hkv, d, bs = 256, 2, 128, 16
+    allv = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(bf).view(T, Hkv, d).to(gpu)
+    qkv = torch.cat([torch.zeros(T, Hkv, d, dtype=bf, device=gpu), allv, allv], 1).view(T, -1)
+    slots = torch.arange(T, device=gpu)
+    shape = (T // bs, Hkv, bs, d)
+    caches = [torch.zeros(shape, dtype=torch.float8_e4m3fn, device=gpu) for _ in range(4)]
+    if packed:
+        caches[0] = torch.zeros((T // bs, Hkv, bs // 2, d, 2), dtype=torch.float8_e4m3fn, device=gpu)
+    kw = {} if mode == N.QUANT_NONE else dict(
+        quant_mode=mode, k_scale=torch.tensor([0.37, 3.1], device=gpu),
+        v_scale=torch.tensor([0.011, 57.0], device=gpu), scale_per_head=True)
+    k_out = torch.empty(T, Hkv, d, dtype=bf, device=gpu)
+    K.qkv_epilogue(qkv, Hkv, Hkv, d, k_out=k_out, slots=slots, k_cache=caches[0],
+                   v_cache=caches[1], k_packed=packed, **kw)
+    K.kv_write(allv, allv, slots, caches[2], caches[3], **kw)
+    want = caches[2].view(torch.uint8)
+    if packed:
+        want = OP.swizzle_packed_k(want.cpu()).to(gpu)
+    assert torch.equal(caches[0].view(torch.uint8).view(want.shape), want)
+    assert torch.equal(caches[1].view(torch.uint8), caches[3].view(torch.uint8))
+    nan = allv.isnan()
+    assert torch.equal(k_out.isnan(), nan)
+    assert torch.equal(k_out.view(torch.int16)[~nan], allv.view(torch.int16)[~nan])

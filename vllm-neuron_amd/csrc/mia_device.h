@@ -101,6 +101,19 @@ MIA_HD uint32_t f32_to_e4m3fn_bits(float x) {
   return sign | code;
 }
 
+// Four codes in one dword, byte order = element order: the same codes as
+// f32_to_e4m3fn_bits, by v_cvt_pk_fp8_f32 (round to nearest even) where all
+// four lie inside +-448, else (past it, NaN) by the integer form.
+MIA_DEV uint32_t e4m3fn_x4(float y0, float y1, float y2, float y3) {
+  if (__builtin_expect(fabsf(y0) <= 448.0f && fabsf(y1) <= 448.0f && fabsf(y2) <= 448.0f &&
+                           fabsf(y3) <= 448.0f, 1)) {
+    const int lo = __builtin_amdgcn_cvt_pk_fp8_f32(y0, y1, 0, false);
+    return (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(y2, y3, lo, true);
+  }
+  return f32_to_e4m3fn_bits(y0) | (f32_to_e4m3fn_bits(y1) << 8) |
+         (f32_to_e4m3fn_bits(y2) << 16) | (f32_to_e4m3fn_bits(y3) << 24);
+}
+
 // e4m3fn -> f32 (exact; NaN codes give NaN).
 MIA_HD float e4m3fn_bits_to_f32(uint32_t b) {
   uint32_t sign = (b & 0x80u) << 24;

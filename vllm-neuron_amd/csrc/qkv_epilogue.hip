@@ -16,7 +16,8 @@
 namespace mia {
 namespace {
 
-MIA_DEV float round_bf16(float x) { return bf16_bits_to_f32(f32_to_bf16_bits(x)); }
+// v_cvt_pk_bf16_f32 and a shift: the integer form is ~8 instructions
+MIA_DEV float round_bf16(float x) { return bf16lo(pack2_bf16(x, 0.f)); }
 
 MIA_DEV int64_t slot_at(const void *slots, int64_t t, int dtype) {
   if (dtype == MIA_DTYPE_I64) return ((const int64_t *)slots)[t];
@@ -33,8 +34,10 @@ MIA_DEV void rotate_pair(float &xa, float &xb, float ca, float sa, float cb, flo
 #pragma clang fp contract(off)
   float ya, yb;
   if (bf16_steps) {
-    ya = round_bf16(round_bf16(xa * ca) - round_bf16(xb * sa));
-    yb = round_bf16(round_bf16(xb * cb) + round_bf16(xa * sb));
+    const uint32_t p = pack2_bf16(xa * ca, xb * sa), q = pack2_bf16(xb * cb, xa * sb);
+    const uint32_t y = pack2_bf16(bf16lo(p) - bf16hi(p), bf16lo(q) + bf16hi(q));
+    ya = bf16lo(y);
+    yb = bf16hi(y);
   } else {
     const float p0 = xa * ca, p1 = xb * sa, p2 = xb * cb, p3 = xa * sb;
     ya = p0 - p1;
@@ -52,7 +55,15 @@ MIA_DEV void rotate_pair(float &xa, float &xb, float ca, float sa, float cb, flo
 // Loads and stores are 8 or 16 bytes wide.  The lanes of a row are an
 // aligned group, so its norm reduction is a butterfly of xor shuffles inside
 // the group.
-constexpr int kMaxHpg = 4;  // head rows per lane group at most (the host splits beyond)
+//
+// Bound by instruction issue and, since every wave loads, computes and stores
+// at about the same time, by phases that hardly overlap.  2048 tokens of 48 q /
+// 8 kv heads, d = 128, packed FP8 cache write (56 MB with Q in place): 28.4 us
+// with bf16 and e4m3fn rounded in integer code and K / V also stored as rows,
+// 22.9 with v_cvt_pk_bf16_f32 and without idle norm shuffles, 21.8 with
+// v_cvt_pk_fp8_f32 and K / V to the cache alone, 20.2 with two rows per group
+// instead of four (one: 22.8; the cos / sin loads then weigh more).
+constexpr int kMaxHpg = 2;  // head rows per lane group at most (the host splits beyond)
 
 template <int D>
 __global__ __launch_bounds__(256) void qkv_epilogue_kernel(mia_qkv_epilogue_args a, int hpg,
@@ -135,6 +146,7 @@ __global__ __launch_bounds__(256) void qkv_epilogue_kernel(mia_qkv_epilogue_args
     // x <- bf16(x * rsqrt(mean(x^2) + eps) * gamma + beta) when enabled for this kind
     auto norm = [&](int flags, float eps, const float *gq, const float *gk, const float *bq,
                     const float *bk) {
+      if (flags == 0) return;  // uniform: no sum, no shuffles
       float ss = 0.f;
 #pragma unroll
       for (int i = 0; i < NP; ++i) ss += xa[i] * xa[i] + xb[i] * xb[i];
@@ -166,29 +178,32 @@ __global__ __launch_bounds__(256) void qkv_epilogue_kernel(mia_qkv_epilogue_args
       }
     }
     norm(a.norm_post, a.eps_post, a.gamma_post_q, a.gamma_post_k, a.beta_post_q, a.beta_post_k);
-    uint32_t ba[NP], bb[NP];
+    if (kind == 0) {
 #pragma unroll
-    for (int i = 0; i < NP; ++i) {
-      if (kind == 0) {
+      for (int i = 0; i < NP; ++i) {
         xa[i] *= a.q_scale;
         xb[i] *= a.q_scale;
       }
-      ba[i] = f32_to_bf16_bits(xa[i]);
-      bb[i] = f32_to_bf16_bits(xb[i]);
     }
-
-    // bf16 row store of the 4 pairs (elements contiguous in memory)
+    // the row's bf16 words in memory order: elements 8j..8j+7 interleaved, 4j..
+    // and d/2 + 4j.. in the half split
+    u32x4_t bw;
+    if (inter) {
+#pragma unroll
+      for (int i = 0; i < NP; ++i) bw[i] = pack2_bf16(xa[i], xb[i]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        bw[i] = pack2_bf16(xa[2 * i], xa[2 * i + 1]);
+        bw[2 + i] = pack2_bf16(xb[2 * i], xb[2 * i + 1]);
+      }
+    }
     auto store_row = [&](uint16_t *dst) {
       if (inter) {
-        u32x4_t w;
-#pragma unroll
-        for (int i = 0; i < NP; ++i) w[i] = ba[i] | (bb[i] << 16);
-        *reinterpret_cast<u32x4_t *>(dst + 8 * j) = w;
+        *reinterpret_cast<u32x4_t *>(dst + 8 * j) = bw;
       } else {
-        *reinterpret_cast<u32x2_t *>(dst + 4 * j) =
-            u32x2_t{ba[0] | (ba[1] << 16), ba[2] | (ba[3] << 16)};
-        *reinterpret_cast<u32x2_t *>(dst + P + 4 * j) =
-            u32x2_t{bb[0] | (bb[1] << 16), bb[2] | (bb[3] << 16)};
+        *reinterpret_cast<u32x2_t *>(dst + 4 * j) = u32x2_t{bw[0], bw[1]};
+        *reinterpret_cast<u32x2_t *>(dst + P + 4 * j) = u32x2_t{bw[2], bw[3]};
       }
     };
 
@@ -227,9 +242,8 @@ __global__ __launch_bounds__(256) void qkv_epilogue_kernel(mia_qkv_epilogue_args
       const float *sc = kind == 1 ? a.k_scale : a.v_scale;
       s = sc[a.scale_per_head ? h : 0];
     }
-    auto code = [&](uint32_t bits) -> uint32_t {
-      const float x = bf16_bits_to_f32(bits);
-      if (a.quant_mode == MIA_QUANT_NONE) return f32_to_e4m3fn_bits(x);
+    auto quant = [&](float x) -> float {
+      if (a.quant_mode == MIA_QUANT_NONE) return x;
       float y;
       if (a.quant_mode == MIA_QUANT_MUL_BF16) y = round_bf16(x * s);
       else if (a.quant_mode == MIA_QUANT_DIV_F32) y = x / s;
@@ -237,26 +251,30 @@ __global__ __launch_bounds__(256) void qkv_epilogue_kernel(mia_qkv_epilogue_args
       // torch.clamp keeps NaN; fminf/fmaxf would drop it
       if (y > a.fp8_max) y = a.fp8_max;
       if (y < a.fp8_min) y = a.fp8_min;
-      return f32_to_e4m3fn_bits(y);
+      return y;
     };
-    uint32_t ca[NP], cb[NP];
+    // codes of the elements in the order of bw: dword m holds elements of
+    // words 2m and 2m + 1
+    uint32_t c4[2];
 #pragma unroll
-    for (int i = 0; i < NP; ++i) { ca[i] = code(ba[i]); cb[i] = code(bb[i]); }
+    for (int m = 0; m < 2; ++m) {
+      const float y0 = quant(bf16lo(bw[2 * m])), y1 = quant(bf16hi(bw[2 * m]));
+      const float y2 = quant(bf16lo(bw[2 * m + 1])), y3 = quant(bf16hi(bw[2 * m + 1]));
+      c4[m] = e4m3fn_x4(y0, y1, y2, y3);
+    }
     uint8_t *c8 = (uint8_t *)cache + base;
+    const int e0 = inter ? 8 * j : 4 * j, e1 = inter ? 8 * j + 4 : P + 4 * j;
     if (packed) {  // element e at 2 e (the pair partner's bytes interleave)
 #pragma unroll
-      for (int i = 0; i < NP; ++i) {
-        c8[2 * ea(i)] = (uint8_t)ca[i];
-        c8[2 * eb(i)] = (uint8_t)cb[i];
+      for (int i = 0; i < 4; ++i) {
+        c8[2 * (e0 + i)] = (uint8_t)(c4[0] >> (8 * i));
+        c8[2 * (e1 + i)] = (uint8_t)(c4[1] >> (8 * i));
       }
     } else if (inter) {
-      *reinterpret_cast<u32x2_t *>(c8 + 8 * j) =
-          u32x2_t{ca[0] | (cb[0] << 8) | (ca[1] << 16) | (cb[1] << 24),
-                  ca[2] | (cb[2] << 8) | (ca[3] << 16) | (cb[3] << 24)};
+      *reinterpret_cast<u32x2_t *>(c8 + e0) = u32x2_t{c4[0], c4[1]};
     } else {
-      *reinterpret_cast<uint32_t *>(c8 + 4 * j) = ca[0] | (ca[1] << 8) | (ca[2] << 16) | (ca[3] << 24);
-      *reinterpret_cast<uint32_t *>(c8 + P + 4 * j) =
-          cb[0] | (cb[1] << 8) | (cb[2] << 16) | (cb[3] << 24);
+      *reinterpret_cast<uint32_t *>(c8 + e0) = c4[0];
+      *reinterpret_cast<uint32_t *>(c8 + e1) = c4[1];
     }
   };
   // one copy of the row code (the rows shift down the loaded registers): the

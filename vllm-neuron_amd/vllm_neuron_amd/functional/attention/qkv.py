@@ -213,8 +213,9 @@ def qkv_proj(
                           v_scale=v_scale.reshape(-1)[:1],
                           fp8_min=-448.0 if fp8_min is None else float(fp8_min),
                           fp8_max=448.0 if fp8_max is None else float(fp8_max))
-        K.qkv_epilogue(flat, Hq, Hkv, d, q_out=heads[:, :Hq], k_out=heads[:, Hq:Hq + Hkv],
-                       v_out=heads[:, Hq + Hkv:], **kw)
+        if not use_block_kv:  # with the cache write K and V are read from the cache alone
+            kw.update(k_out=heads[:, Hq:Hq + Hkv], v_out=heads[:, Hq + Hkv:])
+        K.qkv_epilogue(flat, Hq, Hkv, d, q_out=heads[:, :Hq], **kw)
         if use_block_kv:
             return out[:, :, :Hq * d], k_cache, v_cache
 
