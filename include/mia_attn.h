@@ -339,7 +339,11 @@ typedef struct {
   void *workspace;
   size_t workspace_bytes;
   int32_t split_tokens;
-  int32_t _pad0;
+  /* Below head_dim and a multiple of 8: the q and out rows hold only this many
+   * channels (none past it is read or written) and the cache rows are zero
+   * from there on, i.e. the caller padded a narrower K and V to head_dim.
+   * Any other value (0): every row holds head_dim channels. */
+  int32_t head_dim_used;
   /* Generalised visibility for dense attention (attention_cte.py:47-186,
    * flash_attention :189-343); all zero / NULL keeps the rule above.
    *   kv_len      device [num_seqs]: keys [0, kv_len) exist (NULL: prior + S_q).

@@ -198,3 +198,24 @@ def test_stage_rows_exact(gpu, H, S, P, extra, D, Dp, layout):
         src = rows.transpose(1, 2).contiguous().to(gpu).transpose(1, 2)
     got = K.stage_rows(src, prior.to(gpu) if P else None, P, Lp, Dp)
     assert torch.equal(got.cpu(), exp)
+
+
+@pytest.mark.parametrize("D", [48, 72, 80, 88, 96, 104])
+@pytest.mark.parametrize("B,B_kv,S,causal", [(2, 2, 65, True), (4, 2, 1030, False), (8, 2, 700, True)])
+def test_unpadded_queries_and_outputs(gpu, D, B, B_kv, S, causal):
+    """Head dims between the compiled widths: q and the output keep their own
+    width (the products stop at 80 or 96 channels, or run all 64 / 128), so
+    nothing past a q row's channels is read: the gap between q rows is NaN.
+    Tile edges, few row tiles (4-wave workgroups) and split key ranges."""
+    g = torch.Generator().manual_seed(D + S)
+    q = torch.full((B, S, D + 8), float("nan"), dtype=torch.bfloat16)
+    q[:, :, :D] = torch.randn(B, S, D, generator=g).to(torch.bfloat16)
+    k = torch.randn(B_kv, D, S, generator=g).to(torch.bfloat16)
+    v = torch.randn(B_kv, S, D, generator=g).to(torch.bfloat16)
+    out = flash_attention(q.to(gpu)[:, :, :D], k.to(gpu), v.to(gpu), causal_mask=causal)
+    assert out.shape == (B, S, D)
+    sc = q[:, :, :D].double() @ k.double().repeat_interleave(B // B_kv, 0) * D ** -0.5
+    if causal:
+        sc = sc.masked_fill(~torch.ones(S, S, dtype=torch.bool).tril(), float("-inf"))
+    ref = torch.softmax(sc, -1) @ v.double().repeat_interleave(B // B_kv, 0)
+    assert (out.cpu().double() - ref).abs().max().item() <= 2e-2

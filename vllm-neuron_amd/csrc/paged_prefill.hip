@@ -80,6 +80,7 @@ struct PrefillKParams {
   int num_tokens;
   uint16_t *out;
   int32_t os_t, os_h;
+  int d_used;     // channels of a q and out row; the cache's are zero past it
   // split-K over keys (nsplit == 1: off)
   uint8_t *ws;    // [num_seqs, Hkv, rows_max, nsplit] partial rows (part_bytes(D) each)
   int nsplit;     // chunks per row tile at most (grid z = nsplit * num_seqs)
@@ -428,6 +429,7 @@ MIA_DEV void store_final(const PrefillKParams &p, const f32x16_t (&acc_o)[D / 32
 #pragma unroll
       for (int e4 = 0; e4 < 4; ++e4) {
         const int d0 = db * 32 + e4 * 8 + half * 4;
+        if (d0 >= p.d_used) continue;
         const u32x2_t w = {pack2_bf16(acc_o[db][e4 * 4] * inv, acc_o[db][e4 * 4 + 1] * inv),
                            pack2_bf16(acc_o[db][e4 * 4 + 2] * inv, acc_o[db][e4 * 4 + 3] * inv)};
         *reinterpret_cast<u32x2_t *>(op + d0) = w;
@@ -704,7 +706,8 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillKParams p) {
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ++ks) {
       u32x4_t w = {0u, 0u, 0u, 0u};  // zero query: uniform row, scores 0
-      if (row_ok && !uni) w = *reinterpret_cast<const u32x4_t *>(qp + ks * 16 + half * 8);
+      if (row_ok && !uni && ks * 16 + half * 8 < p.d_used)
+        w = *reinterpret_cast<const u32x4_t *>(qp + ks * 16 + half * 8);
       qf[ks] = scale_q8(w, scale2);
     }
   }
@@ -928,9 +931,16 @@ static_assert(waitcnt_vm(4) == 0xF74 && waitcnt_vm(0) == 0xF70, "vmcnt encoding"
 // workgroups at three per CU measured 202-209 us: the SIMDs run at the power
 // limit (the clock falls from 2.3 to 1.6 GHz as products and exponentials
 // overlap), so more waves do not help.  Reading ahead at d = 128 costs 1-5 %.
-template <int D, int WAVES, int STAGES, bool FP8, bool PK>
+//
+// DU < D: a cache zero-padded from a head dim of at most DU; the products stop
+// there (QK steps of 16 channels, O^T blocks of 32).  16 heads x 4096 tokens,
+// d = 80, not causal: 133 us with all 128 channels, 105 with 80 (86 GFLOP of the
+// useful channels; with the staging of q left out too the call went 141 -> 113).
+// Reading fragments ahead, as at d = 64, measured 2 % slower.
+template <int D, int WAVES, int STAGES, bool FP8, bool PK, int DU = D>
 __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void prefill_dma_kernel(
     PrefillKParams p) {
+  static_assert(DU == D || (D == 128 && !FP8 && DU > 64 && DU % 16 == 0), "padded head dims");
   static_assert(D == 128 || D == 64, "256- or 128-byte rows");
   static_assert((WAVES == 8 || WAVES == 4) && (STAGES == 2 || STAGES == 3), "ring shape");
   static_assert(!FP8 || (D == 128 && WAVES == 8 && STAGES == 3), "FP8 ring: one chunk per thread");
@@ -938,8 +948,8 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void prefill_dma_kernel(
   constexpr int kDmaWaves = WAVES;
   constexpr int kDmaRows = dma_rows(WAVES);
   constexpr int kDmaIds = dma_ids(WAVES);
-  constexpr int KSTEPS = D / 16;
-  constexpr int DBLK = D / 32;
+  constexpr int KSTEPS = DU / 16;
+  constexpr int DBLK = (DU + 31) / 32;
   constexpr int ROWB = D * 2;          // bytes per K/V row
   constexpr int TILEB = kKT * ROWB;    // bytes per K (or V) tile
   constexpr int NJ = TILEB / 1024 / kDmaWaves;  // DMA instructions per thread per tile (K, V each)
@@ -1046,7 +1056,9 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void prefill_dma_kernel(
                          (int64_t)(row_ok ? hq : 0) * p.qs_h;
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ++ks)
-      qw[ks] = *reinterpret_cast<const u32x4_t *>(qp + ks * 16 + half * 8);
+      qw[ks] = ks * 16 + half * 8 < p.d_used
+                   ? *reinterpret_cast<const u32x4_t *>(qp + ks * 16 + half * 8)
+                   : u32x4_t{0u, 0u, 0u, 0u};
   }
   if (tid < n_blk) ids_lds[tid] = blk_id(bt0);
   for (int i = tid + WAVES * 64; i < n_blk; i += WAVES * 64)
@@ -1374,7 +1386,7 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void prefill_dma_kernel(
   lds_u8_t *const ob = kv_base + wave * (kRowsW * ROWB);
   if (split && p.even) {
     // fp32 partial, half the row's columns at a time: ROWB bytes per row
-    constexpr int DBP = DBLK / 2;
+    constexpr int DBP = D / 64;
     float *const part = reinterpret_cast<float *>(p.ws);
     const int64_t step = (int64_t)p.nsplit * (part32_bytes(D) / 4);
     const int64_t first = ((int64_t)h * p.rows_max + row0 + wave * kRowsW) * step +
@@ -1385,8 +1397,9 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void prefill_dma_kernel(
       for (int db = 0; db < DBP; ++db)
 #pragma unroll
         for (int e4 = 0; e4 < 4; ++e4) {
+          if (pass * DBP + db >= DBLK) continue;
           const int c = db * 8 + e4 * 2 + half;
-          const f32x16_t &a = acc_o[pass * DBP + db];
+          const f32x16_t &a = acc_o[pass * DBP + db < DBLK ? pass * DBP + db : 0];
           *(__attribute__((address_space(3))) f32x4_t *)(ob + rl * ROWB +
                                                          ((c ^ (rl & (CH - 1))) << 4)) =
               f32x4_t{a[e4 * 4] * vscale, a[e4 * 4 + 1] * vscale, a[e4 * 4 + 2] * vscale,
@@ -1399,7 +1412,8 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void prefill_dma_kernel(
         const f32x4_t v = *(const __attribute__((address_space(3))) f32x4_t *)(
             ob + rl2 * ROWB + ((ch ^ (rl2 & (CH - 1))) << 4));
         const int r2 = row0 + wave * kRowsW + rl2;
-        if (r2 < rows_total && q_begin + r2 / G < p.num_tokens)
+        if (r2 < rows_total && q_begin + r2 / G < p.num_tokens &&
+            pass * (D / 2) + ch * 4 < p.d_used)
           *reinterpret_cast<f32x4_t *>(part + first + rl2 * step + pass * (D / 2) + ch * 4) = v;
       }
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // read before the next pass writes
@@ -1432,7 +1446,7 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void prefill_dma_kernel(
         ob + rl2 * ROWB + ((ch ^ (rl2 & (CH - 1))) << 4));
     const int r2 = row0 + wave * kRowsW + rl2;
     const int pos2 = r2 / G;
-    if (r2 >= rows_total || q_begin + pos2 >= p.num_tokens) continue;
+    if (r2 >= rows_total || q_begin + pos2 >= p.num_tokens || ch * 8 >= p.d_used) continue;
     if (split) {
       uint8_t *w = p.ws + ((((int64_t)seq * p.Hkv + h) * p.rows_max + r2) * p.nsplit + sp) *
                               (int64_t)part_bytes(D);
@@ -1520,7 +1534,7 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(PrefillKParams p) 
       }
     }
     const float inv = L > 0.f ? 1.0f / L : 0.f;
-    if (ok && q_begin + pos_r < p.num_tokens) {
+    if (ok && q_begin + pos_r < p.num_tokens && c8 < p.d_used) {
       uint16_t *op = p.out + (int64_t)(q_begin + pos_r) * p.os_t + (int64_t)hq * p.os_h + c8;
       // two 8-byte stores: the output is only 8-byte aligned
       *reinterpret_cast<u32x2_t *>(op) =
@@ -1590,7 +1604,7 @@ __global__ __launch_bounds__(256) void prefill_merge32_kernel(PrefillKParams p) 
     }
     M = Mn;
   }
-  if (q_begin + pos_r >= p.num_tokens) return;
+  if (q_begin + pos_r >= p.num_tokens || c8 >= p.d_used) return;
   const float inv = L > 0.f ? 1.0f / L : 0.f;
   uint16_t *op = p.out + (int64_t)(q_begin + pos_r) * p.os_t + (int64_t)hq * p.os_h + c8;
   // two 8-byte stores: the output is only 8-byte aligned
@@ -1616,6 +1630,12 @@ int device_cus() {
     cache[dev] = n;
   }
   return cache[dev];
+}
+
+// Channels of a q / out row (below head_dim: the caller padded the cache).
+int prefill_head_dim_used(const mia_prefill_args &a) {
+  const int u = a.head_dim_used;
+  return u > 0 && u < a.head_dim && u % 8 == 0 ? u : a.head_dim;
 }
 
 bool use_dma_kernel(const mia_prefill_args &a) {
@@ -1820,6 +1840,7 @@ int launch_paged_prefill(const mia_prefill_args &a, const PrefillPlan &pl, hipSt
   kp.os_t = (int32_t)a.out_stride[0];
   kp.os_h = (int32_t)a.out_stride[1];
   kp.ws = (uint8_t *)a.workspace;
+  kp.d_used = prefill_head_dim_used(a);
   kp.nsplit = pl.nsplit;
   kp.ksplit = pl.ksplit;
   kp.even = pl.even ? 1 : 0;
@@ -1850,14 +1871,27 @@ int launch_paged_prefill(const mia_prefill_args &a, const PrefillPlan &pl, hipSt
     hipLaunchKernelGGL((prefill_dma_kernel<64, kDmaWaves, kDmaStages, false, false>), grid,
                        dim3(kDmaWaves * 64), 0, s, kp);
   } else if (pl.dma && pl.dma_waves == 4) {
-    hipLaunchKernelGGL((prefill_dma_kernel<128, 4, 2, false, false>), grid, dim3(4 * 64), 0, s,
-                       kp);
+    if (kp.d_used <= 80)
+      hipLaunchKernelGGL((prefill_dma_kernel<128, 4, 2, false, false, 80>), grid, dim3(4 * 64), 0,
+                         s, kp);
+    else if (kp.d_used <= 96)
+      hipLaunchKernelGGL((prefill_dma_kernel<128, 4, 2, false, false, 96>), grid, dim3(4 * 64), 0,
+                         s, kp);
+    else
+      hipLaunchKernelGGL((prefill_dma_kernel<128, 4, 2, false, false>), grid, dim3(4 * 64), 0, s,
+                         kp);
   } else if (pl.dma) {
     if (fp8 && a.k_packed)
       hipLaunchKernelGGL((prefill_dma_kernel<128, kDmaWaves, kDmaStages, true, true>), grid,
                          dim3(kDmaWaves * 64), 0, s, kp);
     else if (fp8)
       hipLaunchKernelGGL((prefill_dma_kernel<128, kDmaWaves, kDmaStages, true, false>), grid,
+                         dim3(kDmaWaves * 64), 0, s, kp);
+    else if (kp.d_used <= 80)
+      hipLaunchKernelGGL((prefill_dma_kernel<128, kDmaWaves, kDmaStages, false, false, 80>), grid,
+                         dim3(kDmaWaves * 64), 0, s, kp);
+    else if (kp.d_used <= 96)
+      hipLaunchKernelGGL((prefill_dma_kernel<128, kDmaWaves, kDmaStages, false, false, 96>), grid,
                          dim3(kDmaWaves * 64), 0, s, kp);
     else
       hipLaunchKernelGGL((prefill_dma_kernel<128, kDmaWaves, kDmaStages, false, false>), grid,

@@ -426,6 +426,7 @@ def paged_prefill(
     empty_rows_uniform: bool = False,
     k_packed: bool = False,
     compact_kernel: bool = False,
+    padded_cache: bool = False,
 ) -> torch.Tensor:
     """``q [T, Hq, d]`` (any token/head strides) over paged K/V; sequence i
     owns rows ``cu_seqlens_q[i]:cu_seqlens_q[i+1]`` and table row i.
@@ -441,7 +442,8 @@ def paged_prefill(
     visible iff bound_min <= k < bound_max), and ``empty_rows_uniform``
     (a row that sees no key and has no sink averages all keys uniformly).
     ``k_packed``: ``k_cache`` is the packed FP8 layout ``[nb, Hkv, bs/2, d,
-    2]``, read as it lies."""
+    2]``, read as it lies.  ``padded_cache``: q (and the output) are narrower
+    than the cache rows, which are zero past q's head dim (a multiple of 8)."""
     # every tensor whose address reaches a kernel must live on the device
     dev = N.require_gpu(q, cu_seqlens_q, prior_tokens, k_cache, v_cache, block_table, sink,
                         out, workspace, kv_len, bound_min, bound_max)
@@ -452,7 +454,7 @@ def paged_prefill(
     T, Hq, d = q.shape
     ks, hkv, bs, cd, nb = _cache_view(k_cache, packed=k_packed)
     vs, _, _, _, _ = _cache_view(v_cache)
-    if cd != d:
+    if cd != d and not (padded_cache and 0 < d < cd and d % 8 == 0):
         raise ValueError(f"head_dim mismatch: q {d}, cache {cd}")
     if block_table.dim() == 2:
         nblk = block_table.shape[1]
@@ -502,7 +504,8 @@ def paged_prefill(
     a.blocks_per_seq = nblk
     a.num_q_heads = Hq
     a.num_kv_heads = hkv
-    a.head_dim = d
+    a.head_dim = cd
+    a.head_dim_used = d
     a.scale = float(scale)
     a.sliding_window = int(sliding_window or 0)
     a.sink = N.ptr(sk)

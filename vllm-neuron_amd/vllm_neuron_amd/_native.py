@@ -117,7 +117,7 @@ class PrefillArgs(ctypes.Structure):
         ("sink", c_vp), ("k_dequant", c_vp), ("v_dequant", c_vp),
         ("out_dtype", c_i32), ("num_tokens", c_i32), ("out", c_vp), ("out_stride", c_i64 * 3),
         ("workspace", c_vp), ("workspace_bytes", ctypes.c_size_t),
-        ("split_tokens", c_i32), ("_pad0", c_i32),
+        ("split_tokens", c_i32), ("head_dim_used", c_i32),
         ("kv_len", c_vp), ("bound_min", c_vp), ("bound_max", c_vp), ("bound_stride", c_i64 * 2),
         ("non_causal", c_i32), ("q_offset", c_i32), ("empty_rows_uniform", c_i32),
         ("compact_kernel", c_i32),

@@ -159,9 +159,11 @@ def flash_attention(
         kv_len = P_dev + S_k
         qpos0 = P_dev + _device_i32(cp_offset, dev) if cp_offset is not None else P_dev
 
-    # queries [T = S_q, Hq = B, Dp] and the output through strided views
-    qp = qr if _kernel_rows_ok(qr, Dp) else K.stage_rows(qr, None, 0, S_q, Dp)
-    out = torch.empty((B, S_q, Dp), dtype=torch.bfloat16, device=dev)
+    # queries [T = S_q, Hq = B, Dq] and the output through strided views; a
+    # head dim that is a multiple of 8 needs no padding there (Dq = D)
+    Dq = D if D % 8 == 0 else Dp
+    qp = qr if _kernel_rows_ok(qr, Dq) else K.stage_rows(qr, None, 0, S_q, Dq)
+    out = torch.empty((B, S_q, Dq), dtype=torch.bfloat16, device=dev)
     q_view = qp.permute(1, 0, 2)
     out_view = out.permute(1, 0, 2)
 
@@ -174,6 +176,7 @@ def flash_attention(
     K.paged_prefill(q_view, cu, qpos0, S_q, k_cache, v_cache, table, scale=float(scale),
                     sliding_window=sliding_window if causal_mask else 0, sink=sk,
                     out=out_view, kv_len=kv_len, non_causal=not causal_mask, q_offset=0,
-                    bound_min=bmin, bound_max=bmax, empty_rows_uniform=True)
-    res = out if Dp == D else out[:, :, :D]
+                    bound_min=bmin, bound_max=bmax, empty_rows_uniform=True,
+                    padded_cache=Dq < Dp)
+    res = out if Dq == D else out[:, :, :D]
     return res.transpose(-2, -1) if tp_out else res
