@@ -530,10 +530,11 @@ int mia_stage_rows(const mia_stage_args *args, mia_stream_t stream);
 /*   Q only     y <- y * q_scale                                              */
 /* V heads pass through.  bf16_steps = 1 rounds every product and sum of the  */
 /* RoPE to bf16 (the reference's bf16 tensor ops); 0 keeps them in fp32      */
-/* (no contraction).  Each norm rounds its output to bf16, as the reference   */
-/* does; outputs are bf16.  The cache write stores the final K and V rows     */
-/* (bf16 copy, or FP8 by quant_mode, clamped to [fp8_min, fp8_max]) at        */
-/* slots[t]; slots outside [0, num_blocks * block_size) are skipped.          */
+/* (no contraction); 2 is 1 with the cos and sin values rounded to bf16       */
+/* first.  Each norm rounds its output to bf16, as the reference does;        */
+/* outputs are bf16.  The cache write stores the final K and V rows (bf16     */
+/* copy, or FP8 by quant_mode, clamped to [fp8_min, fp8_max]) at slots[t];    */
+/* slots outside [0, num_blocks * block_size) are skipped.                    */
 /* ------------------------------------------------------------------------ */
 typedef struct {
   const void *qkv;          /* bf16, d contiguous */

@@ -1,0 +1,92 @@
+"""Which calls skip the dispatcher: ordinary eager ones on ordinary tensors,
+and no call that a mode, transform, trace, subclass or autograd could
+interpose on.  On the GPU, a direct call and the op give the same bits and
+advance the same version counters."""
+import pytest
+import torch
+
+from vllm_neuron_amd import ops
+from vllm_neuron_amd import workloads as W
+
+
+def _contexts():
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch.autograd import forward_ad
+    from torch.overrides import TorchFunctionMode
+
+    class Sub(torch.Tensor):
+        pass
+
+    x = torch.zeros(4)
+    seen = {}
+
+    def note(name, *a):
+        seen[name] = ops._plain(*a)
+        return a[0] * 1
+
+    with FakeTensorMode():
+        seen["fake mode"] = ops._plain(x)
+    with TorchFunctionMode():
+        seen["function mode"] = ops._plain(x)
+    with forward_ad.dual_level():
+        note("forward AD", x)
+    with torch.profiler.profile():
+        note("profiler", x)
+    torch.func.vmap(lambda t: note("vmap", t))(torch.zeros(2, 4))
+    torch.func.grad(lambda t: note("func.grad", t).sum())(x)
+    torch.func.functionalize(lambda t: note("functionalize", t))(x)
+    torch.jit.trace(lambda t: note("jit trace", t), x, check_trace=False)
+    torch.fx.experimental.proxy_tensor.make_fx(lambda t: note("make_fx", t))(x)
+    note("requires grad", x.clone().requires_grad_())
+    note("subclass", x.as_subclass(Sub))
+    note("neg view", torch._neg_view(x))
+    with torch.inference_mode():
+        y = torch.zeros(4)
+    note("inference tensor", y)
+    return seen
+
+
+def test_interposed_calls_take_the_op():
+    import torch.fx.experimental.proxy_tensor  # noqa: F401
+
+    assert {k: v for k, v in _contexts().items() if v} == {}
+
+
+def test_plain_calls_go_direct():
+    x = torch.zeros(4)
+    assert ops._plain(x, None, torch.nn.Parameter(x, requires_grad=False))
+    with torch.no_grad():
+        assert ops._plain(x.clone().requires_grad_())
+    with torch.inference_mode():
+        assert ops._plain(x, torch.zeros(4))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("inference", [False, True])
+def test_direct_calls_equal_the_ops(gpu, monkeypatch, inference):
+    cfg = W.DecodeConfig("t", 3, 8, 2, 128, 32, 50, 500, sink=True, seed=3)
+    pcfg = W.PrefillConfig("t", 1, 8, 2, 128, 32, 70, 96, 96, seed=4)
+    got = []
+    for direct in (True, False):
+        monkeypatch.setattr(ops, "_plain", ops._plain if direct else lambda *t: False)
+        b, p = W.make_decode_batch(cfg, gpu), W.make_prefill_batch(pcfg, gpu)
+        qkv = torch.randn(5, 12 * 128, generator=torch.Generator().manual_seed(1)).to(
+            torch.bfloat16).to(gpu)
+        with torch.inference_mode(inference):
+            out = torch.empty_like(b.q)
+            o = ops.paged_decode(b.q, b.k_new, b.v_new, b.k_cache, b.v_cache, b.block_table,
+                                 softmax_scale=0.1, pos_ids=b.pos, sink=b.sink, out=out,
+                                 write_slots=b.slots)
+            o2 = ops.paged_prefill(p.q, p.cu_seqlens, p.prior, 70, p.k_cache, p.v_cache,
+                                   p.block_table, scale=0.1)
+            ops.kv_write(p.k_new, p.v_new, p.slots, p.k_cache, p.v_cache)
+            q, _, _ = ops.qkv_epilogue(qkv, 8, 2, 128)
+            n = ops.row_norm(qkv, ops.NORM_RMS, 1e-5)
+        tensors = [o, o2, q, n, b.k_cache, b.v_cache, p.k_cache, p.v_cache]
+        versions = [] if inference else [t._version for t in (out, b.k_cache, b.v_cache, p.k_cache,
+                                                              b.q, qkv, n)]
+        versions += [t._version for t in (b.k_cache, p.v_cache, b.block_table)]
+        got.append((tensors, versions))
+    for x, y in zip(got[0][0], got[1][0]):
+        assert torch.equal(x.view(torch.int16), y.view(torch.int16))
+    assert got[0][1] == got[1][1]

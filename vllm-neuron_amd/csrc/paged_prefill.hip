@@ -934,8 +934,8 @@ static_assert(waitcnt_vm(4) == 0xF74 && waitcnt_vm(0) == 0xF70, "vmcnt encoding"
 //
 // DU < D: a cache zero-padded from a head dim of at most DU; the products stop
 // there (QK steps of 16 channels, O^T blocks of 32).  16 heads x 4096 tokens,
-// d = 80, not causal: 133 us with all 128 channels, 105 with 80 (86 GFLOP of the
-// useful channels; with the staging of q left out too the call went 141 -> 113).
+// d = 80, not causal (86 GFLOP of useful channels): 133 us with all 128 channels,
+// 112 with 80; the call, which also no longer stages q, 141 -> 113.
 // Reading fragments ahead, as at d = 64, measured 2 % slower.
 template <int D, int WAVES, int STAGES, bool FP8, bool PK, int DU = D>
 __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void prefill_dma_kernel(

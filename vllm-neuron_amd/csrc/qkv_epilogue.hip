@@ -127,6 +127,16 @@ __global__ __launch_bounds__(256) void qkv_epilogue_kernel(mia_qkv_epilogue_args
     }
   }
 
+  if (a.rope_mode != 0 && a.bf16_steps == 2) {  // the tables are bf16 in effect
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      rc_a[i] = round_bf16(rc_a[i]);
+      rs_a[i] = round_bf16(rs_a[i]);
+      rc_b[i] = round_bf16(rc_b[i]);
+      rs_b[i] = round_bf16(rs_b[i]);
+    }
+  }
+
   auto do_row = [&](int hh, const u32x4_t &w) {
     const int kind = hh < Hq ? 0 : (hh < Hq + Hkv ? 1 : 2);  // Q, K, V
     const int h = kind == 0 ? hh : (kind == 1 ? hh - Hq : hh - Hq - Hkv);

@@ -36,7 +36,8 @@ def _cache_view(cache: torch.Tensor, packed: bool = False):
 
 
 def _arr(ctype, vals):
-    return (ctype * len(vals))(*vals)
+    """Value of a fixed array field: ctypes converts a tuple in C."""
+    return tuple(vals)
 
 
 def _scale_f32(scale: Optional[torch.Tensor], device, need: int = 1,
@@ -784,6 +785,7 @@ def qkv_epilogue(
     scale_per_head: bool = False,
     fp8_min: float = -448.0,
     fp8_max: float = 448.0,
+    round_tables: bool = False,
 ):
     """Per-head norm, RoPE, Q scale and split of a fused projection
     ``qkv [T, (Hq + 2 Hkv) * d]`` (bf16, any row stride), with the optional
@@ -792,7 +794,8 @@ def qkv_epilogue(
     ``cos``/``sin`` are ``[T, n]`` views; pair j of a row uses ``cos[t, j]``
     and ``cos[t, j + cos_hi_off]`` (same for sin).  ``norm_*`` flags: bit 0
     Q heads, bit 1 K heads; ``gamma_*``/``beta_*`` are (Q, K) pairs of
-    ``[d]`` vectors or None.  Returns ``(q_out, k_out, v_out)`` (``[T, H,
+    ``[d]`` vectors or None.  ``round_tables`` (with ``bf16_steps``) rounds the
+    cos / sin values to bf16 first.  Returns ``(q_out, k_out, v_out)`` (``[T, H,
     d]`` bf16; K / V None unless given)."""
     dev = N.require_gpu(qkv)
     if qkv.dtype != torch.bfloat16 or qkv.dim() != 2 or qkv.stride(1) != 1:
@@ -829,7 +832,7 @@ def qkv_epilogue(
         a.cos_stride = _arr(ctypes.c_int64, list(c.stride()))
         a.sin_stride = _arr(ctypes.c_int64, list(s.stride()))
         a.cos_hi_off, a.sin_hi_off = int(cos_hi_off), int(sin_hi_off)
-    a.bf16_steps = 1 if bf16_steps else 0
+    a.bf16_steps = (2 if round_tables else 1) if bf16_steps else 0
     a.norm_pre, a.norm_post = int(norm_pre), int(norm_post)
     a.eps_pre, a.eps_post = float(eps_pre), float(eps_post)
     a.q_scale = float(q_scale)

@@ -296,7 +296,7 @@ def require_gpu(*tensors: torch.Tensor | None) -> torch.device:
     for t in tensors:
         if t is None:
             continue
-        if t.device.type != "cuda":
+        if not t.is_cuda:
             raise RuntimeError(
                 "the MI355X attention path runs on GPU tensors only "
                 f"(got a tensor on {t.device}); there is no CPU fallback"
@@ -311,7 +311,10 @@ def require_gpu(*tensors: torch.Tensor | None) -> torch.device:
 
 
 def stream_ptr(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    # the raw handle of torch's current stream (torch.cuda.current_stream builds a
+    # Stream object around it: ~2 us of a launch's host time)
+    return torch._C._cuda_getCurrentRawStream(
+        torch.cuda.current_device() if device.index is None else device.index)
 
 
 def ptr(t: torch.Tensor | None) -> int | None:

@@ -282,10 +282,12 @@ def attention_decode(
     v = torch.empty_like(k)
     ep = {}
     if cos is not None and sin is not None:
-        # [d/2, B, S] tables cast to bf16 as the reference does; token-major views
-        tab = lambda c: c.to(bf).to(torch.float32).reshape(d_head // 2, T).t()
+        # [d/2, B, S] tables, token-major views, rounded to bf16 as the reference
+        # does (in the kernel; a table of another type from that type)
+        tab = lambda c: (c if c.dtype in (torch.float32, bf) else c.to(bf)).to(
+            torch.float32).reshape(d_head // 2, T).t()
         ep = dict(rope_mode=K.ROPE_HALF if rope_contiguous_layout else K.ROPE_INTERLEAVED,
-                  cos=tab(cos), sin=tab(sin), bf16_steps=True)
+                  cos=tab(cos), sin=tab(sin), bf16_steps=True, round_tables=True)
     if rmsnorm_QK_pre_rope_enabled:
         ep.update(norm_pre=3, eps_pre=rmsnorm_QK_pre_rope_eps,
                   gamma_pre=(rmsnorm_QK_pre_rope_W_Q, rmsnorm_QK_pre_rope_W_K))

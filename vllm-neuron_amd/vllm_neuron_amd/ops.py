@@ -16,6 +16,13 @@ entry point the functionals call is a ``torch.library`` custom op in the
 * the real implementation is the ctypes launch in ``_kernels`` (host
   validation, then one stream-ordered call into ``libmia_attn.so``).
 
+The functionals call most entry points once per layer, and the dispatcher's
+Python kernels (autograd, version counters, backend) take ~15 us of each call.
+A call that nothing could interpose on (``_plain``) therefore goes straight
+to the ctypes launch, with the written tensors' version counters advanced as
+the op does; everything else (tracing, fake or functional tensors, modes,
+transforms, subclasses, tensors that require grad, profiling) takes the op.
+
 The wrappers below keep the keyword signatures of ``_kernels`` and allocate
 outputs the caller did not give with plain torch factories, so the
 functionals trace end to end.  Launch-time options that are not tensors or
@@ -29,8 +36,35 @@ import torch
 from torch import Tensor
 from torch.library import custom_op
 
+from torch.autograd import forward_ad, graph
+
 from . import _kernels as K
 from . import _native as N
+
+_TENSOR_TYPES = (Tensor, torch.nn.Parameter)
+
+
+def _plain(*tensors: Optional[Tensor]) -> bool:
+    """Is this call ordinary eager execution on ordinary tensors, so that
+    the dispatcher would do nothing but run the launch?"""
+    if (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack()
+            or torch._C._len_torch_function_stack() or torch._C._are_functorch_transforms_active()
+            or torch._C._get_tracing_state() is not None or forward_ad._current_level >= 0
+            or torch._C._autograd._profiler_enabled()):
+        return False
+    grad, inference = torch.is_grad_enabled(), torch.is_inference_mode_enabled()
+    for t in tensors:
+        if t is not None and (type(t) not in _TENSOR_TYPES or (grad and t.requires_grad)
+                              or t.is_neg() or (t.is_inference() and not inference)):
+            return False
+    return True
+
+
+def _written(*tensors: Optional[Tensor]) -> None:
+    """Advances the version counters of tensors a direct launch wrote
+    (inference tensors have none)."""
+    graph.increment_version([t for t in tensors if t is not None and not t.is_inference()])
+
 
 # re-exported constants of the kernel wrappers
 NORM_RMS, NORM_LAYER = K.NORM_RMS, K.NORM_LAYER
@@ -57,6 +91,12 @@ def _(k_src, v_src, slots, k_cache, v_cache, k_packed, quant_mode, k_scale, v_sc
 
 def kv_write(k_src, v_src, slots, k_cache, v_cache, *, k_packed=False, quant_mode=N.QUANT_NONE,
              k_scale=None, v_scale=None, scale_per_head=False) -> None:
+    if _plain(k_src, v_src, slots, k_cache, v_cache, k_scale, v_scale):
+        K.kv_write(k_src, v_src, slots, k_cache, v_cache, k_packed=bool(k_packed),
+                   quant_mode=int(quant_mode), k_scale=k_scale, v_scale=v_scale,
+                   scale_per_head=bool(scale_per_head))
+        _written(k_cache, v_cache)
+        return
     _kv_write(k_src, v_src, slots, k_cache, v_cache, bool(k_packed), int(quant_mode), k_scale,
               v_scale, bool(scale_per_head))
 
@@ -128,6 +168,9 @@ def _(rows, prior, prior_rows_dev, prior_rows, out_rows, out_dim):
 
 def stage_rows(rows, prior, prior_rows: int, out_rows: int, out_dim: int,
                prior_rows_dev=None) -> Tensor:
+    if _plain(rows, prior, prior_rows_dev):
+        return K.stage_rows(rows, prior, int(prior_rows), int(out_rows), int(out_dim),
+                            prior_rows_dev)
     return _stage_rows(rows, prior, prior_rows_dev, int(prior_rows), int(out_rows), int(out_dim))
 
 
@@ -302,6 +345,12 @@ def paged_decode(q, k_new, v_new, k_cache, v_cache, block_table, *, softmax_scal
               active_mask, full_mask, sink, k_dequant, v_dequant, k_quant, v_quant)
     scal = (float(softmax_scale), int(mask_block_len), int(quant_mode), bool(quant_per_head),
             int(split_tokens), bool(k_packed), bool(no_alloc))
+    if _plain(*common, write_slots):
+        _decode_launch(*common, write_slots, *scal, bool(write_private))
+        _written(out, workspace)
+        if write_slots is not None:
+            _written(k_cache, v_cache)
+        return out
     if write_slots is None:
         _paged_decode(*common, *scal)
     else:
@@ -345,6 +394,18 @@ def paged_prefill(q, cu_seqlens_q, prior_tokens, max_seqlen_q: int, k_cache, v_c
                   padded_cache: bool = False) -> Tensor:
     if out is None:
         out = q.new_empty(q.shape, dtype=torch.bfloat16)
+    if _plain(q, cu_seqlens_q, prior_tokens, k_cache, v_cache, block_table, out, workspace, sink,
+              k_dequant, v_dequant, kv_len, bound_min, bound_max):
+        K.paged_prefill(q, cu_seqlens_q, prior_tokens, int(max_seqlen_q), k_cache, v_cache,
+                        block_table, scale=float(scale), sliding_window=int(sliding_window or 0),
+                        sink=sink, k_dequant=k_dequant, v_dequant=v_dequant, out=out,
+                        split_tokens=int(split_tokens), workspace=workspace, kv_len=kv_len,
+                        non_causal=bool(non_causal), q_offset=int(q_offset),
+                        bound_min=bound_min, bound_max=bound_max,
+                        empty_rows_uniform=bool(empty_rows_uniform), k_packed=bool(k_packed),
+                        compact_kernel=bool(compact_kernel), padded_cache=bool(padded_cache))
+        _written(out, workspace)
+        return out
     _paged_prefill(q, cu_seqlens_q, prior_tokens, k_cache, v_cache, block_table, out, workspace,
                    sink, k_dequant, v_dequant, kv_len, bound_min, bound_max, int(max_seqlen_q),
                    float(scale), int(sliding_window or 0), int(split_tokens), bool(non_causal),
@@ -370,7 +431,8 @@ def _qkv_epilogue(qkv: Tensor, q_out: Tensor, k_out: Optional[Tensor], v_out: Op
                   head_dim: int, rope_mode: int, cos_hi_off: int, sin_hi_off: int,
                   bf16_steps: bool, norm_pre: int, eps_pre: float, norm_post: int,
                   eps_post: float, q_scale: float, k_packed: bool, quant_mode: int,
-                  scale_per_head: bool, fp8_min: float, fp8_max: float) -> None:
+                  scale_per_head: bool, fp8_min: float, fp8_max: float,
+                  round_tables: bool = False) -> None:
     K.qkv_epilogue(qkv, num_q_heads, num_kv_heads, head_dim, rope_mode=rope_mode, cos=cos,
                    sin=sin, cos_hi_off=cos_hi_off, sin_hi_off=sin_hi_off, bf16_steps=bf16_steps,
                    norm_pre=norm_pre, eps_pre=eps_pre, gamma_pre=(gamma_pre_q, gamma_pre_k),
@@ -379,7 +441,7 @@ def _qkv_epilogue(qkv: Tensor, q_out: Tensor, k_out: Optional[Tensor], v_out: Op
                    q_scale=q_scale, q_out=q_out, k_out=k_out, v_out=v_out, slots=slots,
                    k_cache=k_cache, v_cache=v_cache, k_packed=k_packed, quant_mode=quant_mode,
                    k_scale=k_scale, v_scale=v_scale, scale_per_head=scale_per_head,
-                   fp8_min=fp8_min, fp8_max=fp8_max)
+                   fp8_min=fp8_min, fp8_max=fp8_max, round_tables=round_tables)
 
 
 @_qkv_epilogue.register_fake
@@ -387,7 +449,7 @@ def _(qkv, q_out, k_out, v_out, cos, sin, gamma_pre_q, gamma_pre_k, beta_pre_q, 
       gamma_post_q, gamma_post_k, beta_post_q, beta_post_k, slots, k_cache, v_cache, k_scale,
       v_scale, num_q_heads, num_kv_heads, head_dim, rope_mode, cos_hi_off, sin_hi_off,
       bf16_steps, norm_pre, eps_pre, norm_post, eps_post, q_scale, k_packed, quant_mode,
-      scale_per_head, fp8_min, fp8_max):
+      scale_per_head, fp8_min, fp8_max, round_tables=False):
     return None
 
 
@@ -397,18 +459,34 @@ def qkv_epilogue(qkv, num_q_heads, num_kv_heads, head_dim, *, rope_mode=ROPE_NON
                  eps_post=1e-6, gamma_post=(None, None), beta_post=(None, None), q_scale=1.0,
                  q_out=None, k_out=None, v_out=None, slots=None, k_cache=None, v_cache=None,
                  k_packed=False, quant_mode=N.QUANT_NONE, k_scale=None, v_scale=None,
-                 scale_per_head=False, fp8_min=-448.0, fp8_max=448.0):
+                 scale_per_head=False, fp8_min=-448.0, fp8_max=448.0,
+                 round_tables=False):
     """``_kernels.qkv_epilogue`` through ``mia::qkv_epilogue``; returns
     ``(q_out, k_out, v_out)``."""
     if q_out is None:
         q_out = qkv.new_empty((qkv.shape[0], num_q_heads, head_dim), dtype=torch.bfloat16)
+    if _plain(qkv, q_out, k_out, v_out, cos, sin, *gamma_pre, *beta_pre, *gamma_post, *beta_post,
+              slots, k_cache, v_cache, k_scale, v_scale):
+        K.qkv_epilogue(qkv, int(num_q_heads), int(num_kv_heads), int(head_dim),
+                       rope_mode=int(rope_mode), cos=cos, sin=sin, cos_hi_off=int(cos_hi_off),
+                       sin_hi_off=int(sin_hi_off), bf16_steps=bool(bf16_steps),
+                       norm_pre=int(norm_pre), eps_pre=float(eps_pre), gamma_pre=gamma_pre,
+                       beta_pre=beta_pre, norm_post=int(norm_post), eps_post=float(eps_post),
+                       gamma_post=gamma_post, beta_post=beta_post, q_scale=float(q_scale),
+                       q_out=q_out, k_out=k_out, v_out=v_out, slots=slots, k_cache=k_cache,
+                       v_cache=v_cache, k_packed=bool(k_packed), quant_mode=int(quant_mode),
+                       k_scale=k_scale, v_scale=v_scale, scale_per_head=bool(scale_per_head),
+                       fp8_min=float(fp8_min), fp8_max=float(fp8_max),
+                       round_tables=bool(round_tables))
+        _written(q_out, k_out, v_out, k_cache, v_cache)
+        return q_out, k_out, v_out
     _qkv_epilogue(qkv, q_out, k_out, v_out, cos, sin, gamma_pre[0], gamma_pre[1], beta_pre[0],
                   beta_pre[1], gamma_post[0], gamma_post[1], beta_post[0], beta_post[1], slots,
                   k_cache, v_cache, k_scale, v_scale, int(num_q_heads), int(num_kv_heads),
                   int(head_dim), int(rope_mode), int(cos_hi_off), int(sin_hi_off),
                   bool(bf16_steps), int(norm_pre), float(eps_pre), int(norm_post),
                   float(eps_post), float(q_scale), bool(k_packed), int(quant_mode),
-                  bool(scale_per_head), float(fp8_min), float(fp8_max))
+                  bool(scale_per_head), float(fp8_min), float(fp8_max), bool(round_tables))
     return q_out, k_out, v_out
 
 
@@ -426,6 +504,9 @@ def _(x, gamma, beta, add0, add1, mode, eps, dim_actual):
 
 def row_norm(x, mode: int, eps: float, gamma=None, beta=None, *, add0=None, add1=None,
              dim_actual: int = 0) -> Tensor:
+    if _plain(x, gamma, beta, add0, add1):
+        return K.row_norm(x, int(mode), float(eps), gamma, beta, add0=add0, add1=add1,
+                          dim_actual=int(dim_actual))
     return _row_norm(x, gamma, beta, add0, add1, int(mode), float(eps), int(dim_actual))
 
 
