@@ -620,6 +620,34 @@ typedef struct {
 
 int mia_row_norm(const mia_row_norm_args *args, mia_stream_t stream);
 
+/* ------------------------------------------------------------------------ */
+/* Projection of a few rows (decode): out = norm(x) . w, bf16, fp32          */
+/* accumulation; norm = 1 applies the RMS norm of mia_row_norm to the rows   */
+/* first (gamma fp32, or bf16 with gamma_bf16 = 1; NULL: no gamma).          */
+/* Limits (MIA_ERR_NOT_IMPLEMENTED beyond): rows <= 16, k and n multiples of */
+/* 32, contiguous columns, x and a bf16 gamma 16-byte aligned with row       */
+/* strides a multiple of 8, w 4-byte aligned with an even row stride.        */
+/* ------------------------------------------------------------------------ */
+typedef struct {
+  const void *x; /* [rows, k] */
+  int64_t x_stride;
+  const void *w; /* [k, n] */
+  int64_t w_stride;
+  void *out; /* [rows, n] */
+  int64_t out_stride;
+  int32_t rows;
+  int32_t k;
+  int32_t n;
+  int32_t norm;
+  const void *gamma; /* [k] or NULL */
+  int32_t gamma_bf16;
+  int32_t dim_actual; /* elements the mean divides by (0: k) */
+  float eps;
+  int32_t _pad0;
+} mia_skinny_linear_args;
+
+int mia_skinny_linear(const mia_skinny_linear_args *args, mia_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -461,3 +461,60 @@ def test_epilogue_fp8_codes_of_every_bf16_value(gpu, mode, packed):
     nan = allv.isnan()
     assert torch.equal(k_out.isnan(), nan)
     assert torch.equal(k_out.view(torch.int16)[~nan], allv.view(torch.int16)[~nan])
+
+
+@pytest.mark.parametrize("T,Kd,Nd", [(1, 32, 32), (3, 480, 64), (4, 2048, 3072), (15, 2880, 96),
+                                     (16, 4096, 192), (16, 544, 1088), (7, 8224, 32),
+                                     (2, 64, 8192)])
+@pytest.mark.parametrize("norm", ["none", "rms", "gamma32", "gamma16", "actual"])
+def test_skinny_linear(gpu, T, Kd, Nd, norm):
+    """Fewest and most rows, one k step and shares of unequal or no steps,
+    against float64 of the same operands (the normalised rows rounded to bf16
+    as the kernel rounds them).  Bound: the output's bf16 rounding, 2^-9 of
+    the value, and for the norm the rounding of every operand, 2^-9 each with
+    independent signs: sqrt(K) 2^-9 rms(x w) / sqrt 3, taken six times."""
+    g = torch.Generator().manual_seed(T + Kd)
+    xb = torch.randn(T, Kd + 8, generator=g).to(bf)
+    wb = (torch.randn(Kd, Nd + 2, generator=g) * Kd ** -0.5).to(bf)
+    x, w = xb.to(gpu)[:, :Kd], wb.to(gpu)[:, :Nd]   # strided rows
+    gam = torch.rand(Kd, generator=g) + 0.5
+    kw = {"none": {}, "rms": dict(norm=True, eps=1e-5),
+          "gamma32": dict(norm=True, eps=1e-5, gamma=gam.to(gpu)),
+          "gamma16": dict(norm=True, eps=1e-5, gamma=gam.to(bf).to(gpu)),
+          "actual": dict(norm=True, eps=1e-3, dim_actual=Kd - 8)}[norm]
+    got = K.skinny_linear(x, w, **kw).cpu().double()
+    xd, wd = xb[:, :Kd].double(), wb[:, :Nd].double()
+    if kw:
+        n = kw.get("dim_actual", Kd)
+        xd = xd * torch.rsqrt(xd.pow(2).sum(1, keepdim=True) / n + kw["eps"])
+        if "gamma" in kw:
+            xd = xd * kw["gamma"].cpu().double()
+    ref = xd @ wd
+    noise = 0.0 if not kw else 6 * 2 ** -9 / 3 ** 0.5 * 1.6  # rms(x w) sqrt(K) <= 1.6: gamma <= 1.5
+    assert ((got - ref).abs() <= 2 ** -8 * ref.abs() + noise + 1e-3).all()
+
+
+def test_decode_block_few_rows_equal_many(gpu):
+    """The first rows of a 17-row decode block (library projections) and the
+    same rows as a block of 4 (skinny projections) agree to the rounding of
+    their projections."""
+    B, H, Hq, Hkv, d, bs, nb = 17, 512, 8, 2, 64, 16, 80
+    g = torch.Generator().manual_seed(5)
+    X = torch.randn(B, 1, H, generator=g).to(bf).to(gpu)
+    kw = dict(rmsnorm_X_enabled=True, rmsnorm_X_eps=1e-5,
+              rmsnorm_X_gamma=(torch.rand(H, generator=g) + 0.5).to(bf).to(gpu),
+              W_qkv=(torch.randn(H, (Hq + 2 * Hkv) * d, generator=g) * H ** -0.5).to(bf).to(gpu),
+              W_out=(torch.randn(Hq * d, H, generator=g) * (Hq * d) ** -0.5).to(bf).to(gpu))
+    kc = torch.randn(nb, Hkv, bs, d, generator=g).to(bf).to(gpu)
+    vc = torch.randn(nb, Hkv, bs, d, generator=g).to(bf).to(gpu)
+    table = torch.arange(B * 4, dtype=torch.int32).view(B, 4).to(gpu)
+    pos = torch.randint(1, 60, (B, 1), generator=g).float().to(gpu)
+    ang = torch.rand(d // 2, B, 1, generator=g) * 6
+    outs = []
+    for n in (B, 4):
+        outs.append(attention_decode(X=X[:n].contiguous(), cos=ang.cos()[:, :n].contiguous().to(gpu),
+                                     sin=ang.sin()[:, :n].contiguous().to(gpu),
+                                     active_blocks_table=table[:n].contiguous(), K_cache=kc, V_cache=vc,
+                                     pos_ids=pos[:n].contiguous(), **kw)[0])
+    a, b = outs[0][:4].double(), outs[1].double()
+    assert (a - b).abs().max().item() <= 2e-2 * max(1.0, a.abs().max().item())

@@ -58,6 +58,7 @@ size_t mia_args_size(int which) {
     case 9: return sizeof(mia_stage_args);
     case 10: return sizeof(mia_qkv_epilogue_args);
     case 11: return sizeof(mia_row_norm_args);
+    case 12: return sizeof(mia_skinny_linear_args);
     default: return 0;
   }
 }
@@ -504,6 +505,23 @@ int mia_row_norm(const mia_row_norm_args *a, mia_stream_t stream) {
               "row norm: row strides shorter than the row");
   MIA_REQUIRE(a->rows < (1ll << 31), MIA_ERR_VALUE, "row norm: too many rows");
   return mia::launch_row_norm(*a, (hipStream_t)stream);
+}
+
+int mia_skinny_linear(const mia_skinny_linear_args *a, mia_stream_t stream) {
+  mia::g_last_error.clear();
+  MIA_REQUIRE(a, MIA_ERR_VALUE, "skinny linear: null args");
+  MIA_REQUIRE(a->rows >= 0 && a->k > 0 && a->n > 0 && a->dim_actual >= 0 && a->eps >= 0.f,
+              MIA_ERR_VALUE, "skinny linear: bad shape or eps");
+  if (a->rows == 0) return MIA_OK;
+  MIA_REQUIRE(a->x && a->w && a->out, MIA_ERR_VALUE, "skinny linear: null tensor pointer");
+  MIA_REQUIRE(a->w_stride >= a->n && (a->rows == 1 || (a->x_stride >= a->k && a->out_stride >= a->n)),
+              MIA_ERR_VALUE, "skinny linear: row strides shorter than the row");
+  MIA_REQUIRE(a->rows <= 16 && a->k % 32 == 0 && a->n % 32 == 0, MIA_ERR_NOT_IMPLEMENTED,
+              "skinny linear: rows <= 16, k and n multiples of 32");
+  MIA_REQUIRE(aligned(a->x, 16) && a->x_stride % 8 == 0 && aligned(a->w, 4) &&
+                  a->w_stride % 2 == 0 && (!a->gamma_bf16 || (a->gamma && aligned(a->gamma, 16))),
+              MIA_ERR_NOT_IMPLEMENTED, "skinny linear: unaligned rows");
+  return mia::launch_skinny_linear(*a, (hipStream_t)stream);
 }
 
 static void slot_mapping_one(const mia_slot_mapping_args *a, int64_t t) {

@@ -32,6 +32,7 @@ int launch_scatter_rows(const mia_scatter_rows_args &a, hipStream_t s);
 int launch_stage_rows(const mia_stage_args &a, hipStream_t s);
 int launch_qkv_epilogue(const mia_qkv_epilogue_args &a, hipStream_t s);
 int launch_row_norm(const mia_row_norm_args &a, hipStream_t s);
+int launch_skinny_linear(const mia_skinny_linear_args &a, hipStream_t s);
 
 // Paged decode: split-K plan shared by the workspace query and the launch.
 struct DecodePlan {

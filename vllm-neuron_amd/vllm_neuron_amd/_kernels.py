@@ -936,3 +936,55 @@ def row_norm(x: torch.Tensor, mode: int, eps: float, gamma: Optional[torch.Tenso
     a.beta = b.data_ptr() if b is not None else None
     N.check(N.lib().mia_row_norm(ctypes.byref(a), N.stream_ptr(dev)), "row_norm")
     return out.reshape(shape)
+
+
+def skinny_linear_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Does ``skinny_linear`` take ``x [T, K]`` and ``w [K, N]``, and faster
+    than a library GEMM?  At most 16 rows (one MFMA row block; from 17 rows on
+    the weights would be read twice), whole 32-column and 32-row steps, at most
+    8192 columns (one workgroup of 32 per CU: at 10240 the library is faster,
+    54 against 90 us; at 8192 x 1024 the two are equal).  Strides only:
+    addresses are not known while tracing (see ``skinny_linear``)."""
+    return (x.dim() == 2 and w.dim() == 2 and x.dtype == torch.bfloat16
+            and w.dtype == torch.bfloat16 and 0 < x.shape[0] <= 16 and x.shape[1] == w.shape[0]
+            and x.shape[1] % 32 == 0 and w.shape[1] % 32 == 0 and 0 < w.shape[1] <= 8192
+            and x.shape[1] > 0 and x.stride(1) == 1
+            and w.stride(1) == 1 and x.stride(0) % 8 == 0 and w.stride(0) % 2 == 0
+            and w.stride(0) >= w.shape[1] and (x.shape[0] == 1 or x.stride(0) >= x.shape[1]))
+
+
+def skinny_linear(x: torch.Tensor, w: torch.Tensor, norm: bool = False,
+                  gamma: Optional[torch.Tensor] = None, eps: float = 0.0,
+                  dim_actual: int = 0) -> torch.Tensor:
+    """``x [T, K] @ w [K, N]`` for T <= 16 (``skinny_linear_ok``), with
+    ``norm`` of the RMS-normalised rows (``row_norm`` mode 1).  Rows whose
+    address is not vector aligned are copied first."""
+    dev = N.require_gpu(x, w, gamma)
+    if not skinny_linear_ok(x, w):
+        raise NotImplementedError("skinny_linear: unsupported shapes, strides or dtypes")
+    if x.data_ptr() % 16:
+        x = x.clone()
+    if w.data_ptr() % 4:
+        w = w.clone()
+    T, k = x.shape
+    n = w.shape[1]
+    out = torch.empty((T, n), dtype=torch.bfloat16, device=dev)
+    a = N.SkinnyLinearArgs()
+    a.x, a.x_stride = x.data_ptr(), x.stride(0)
+    a.w, a.w_stride = w.data_ptr(), w.stride(0)
+    a.out, a.out_stride = out.data_ptr(), n
+    a.rows, a.k, a.n = T, k, n
+    if norm:
+        a.norm = 1
+        a.eps = float(eps)
+        a.dim_actual = int(dim_actual)
+        if gamma is not None:
+            if gamma.numel() < k:
+                raise ValueError(f"gamma has {gamma.numel()} entries, needs {k}")
+            if not (gamma.dtype == torch.bfloat16 and gamma.is_contiguous()
+                    and gamma.data_ptr() % 16 == 0):
+                gamma = _scale_f32(gamma, dev, k, "gamma")
+            a.gamma = gamma.data_ptr()
+            a.gamma_bf16 = 1 if gamma.dtype == torch.bfloat16 else 0
+    N.check(N.lib().mia_skinny_linear(ctypes.byref(a), N.stream_ptr(dev)), "skinny_linear")
+    return out

@@ -198,10 +198,20 @@ class RowNormArgs(ctypes.Structure):
     ]
 
 
+class SkinnyLinearArgs(ctypes.Structure):
+    _fields_ = [
+        ("x", c_vp), ("x_stride", c_i64), ("w", c_vp), ("w_stride", c_i64),
+        ("out", c_vp), ("out_stride", c_i64), ("rows", c_i32), ("k", c_i32), ("n", c_i32),
+        ("norm", c_i32), ("gamma", c_vp), ("gamma_bf16", c_i32), ("dim_actual", c_i32),
+        ("eps", c_f32), ("_pad0", c_i32),
+    ]
+
+
+
 ARGS_STRUCTS = {
     0: KvWriteArgs, 1: GatherArgs, 2: MaskArgs, 3: DecodeArgs, 4: PrefillArgs,
     5: SlotMappingArgs, 6: PackedKArgs, 7: SwaTrimArgs, 8: ScatterRowsArgs, 9: StageArgs,
-    10: QkvEpilogueArgs, 11: RowNormArgs,
+    10: QkvEpilogueArgs, 11: RowNormArgs, 12: SkinnyLinearArgs,
 }
 
 # Exported symbols (must match include/mia_attn.h).
@@ -211,7 +221,7 @@ EXPORTS = [
     "mia_paged_decode", "mia_prefill_workspace_bytes", "mia_paged_prefill", "mia_slot_mapping",
     "mia_slot_mapping_host", "mia_remap_null_block", "mia_swa_trim",
     "mia_packed_k_convert", "mia_scatter_rows", "mia_stage_rows", "mia_qkv_epilogue",
-    "mia_row_norm", "mia_paged_decode_noalloc",
+    "mia_row_norm", "mia_skinny_linear", "mia_paged_decode_noalloc",
 ]
 
 # Static scratch capacity of mia_paged_decode_noalloc (include/mia_attn.h).
@@ -233,7 +243,8 @@ def _declare(lib: ctypes.CDLL) -> None:
                      ("mia_paged_prefill", PrefillArgs), ("mia_slot_mapping", SlotMappingArgs),
                      ("mia_swa_trim", SwaTrimArgs), ("mia_packed_k_convert", PackedKArgs),
                      ("mia_scatter_rows", ScatterRowsArgs), ("mia_stage_rows", StageArgs),
-                     ("mia_qkv_epilogue", QkvEpilogueArgs), ("mia_row_norm", RowNormArgs)):
+                     ("mia_qkv_epilogue", QkvEpilogueArgs), ("mia_row_norm", RowNormArgs),
+                     ("mia_skinny_linear", SkinnyLinearArgs)):
         fn = getattr(lib, name)
         fn.argtypes = [P(st), c_vp]
         fn.restype = c_i32

@@ -269,11 +269,15 @@ def attention_decode(
     T = B * S_tkg
     bf = torch.bfloat16
     hidden = X
-    if rmsnorm_X_enabled:
-        eps = rmsnorm_X_eps if rmsnorm_X_eps is not None else 1e-3
-        g = None if rmsnorm_X_gamma is None else rmsnorm_X_gamma.reshape(-1)
+    eps = rmsnorm_X_eps if rmsnorm_X_eps is not None else 1e-3
+    g = None if rmsnorm_X_gamma is None else rmsnorm_X_gamma.reshape(-1)
+    few = bias_qkv is None and K.skinny_linear_ok(X.reshape(T, H), W_qkv)
+    if rmsnorm_X_enabled and not few:
         hidden = K.row_norm(X, K.NORM_RMS, eps, g, dim_actual=X_hidden_dim_actual or 0)
-    if bias_qkv is not None:
+    if few:  # norm and projection in one launch
+        qkv = K.skinny_linear(X.reshape(T, H), W_qkv, rmsnorm_X_enabled, g, eps,
+                              X_hidden_dim_actual or 0)
+    elif bias_qkv is not None:
         qkv = torch.addmm(bias_qkv.reshape(1, -1).to(bf), hidden.reshape(T, H), W_qkv.to(bf))
     else:
         qkv = torch.mm(hidden.reshape(T, H), W_qkv.to(bf))
@@ -330,7 +334,9 @@ def attention_decode(
     # ---- stage 9: output projection (library GEMM)
     if W_out is not None:
         a2 = attn.reshape(B * S_tkg, q_heads * d_head)
-        if bias_out is not None:
+        if bias_out is None and K.skinny_linear_ok(a2, W_out):
+            output = K.skinny_linear(a2, W_out)
+        elif bias_out is not None:
             output = torch.addmm(bias_out.reshape(1, -1).to(a2.dtype), a2, W_out.to(a2.dtype))
         else:
             output = a2 @ W_out

@@ -510,9 +510,37 @@ def row_norm(x, mode: int, eps: float, gamma=None, beta=None, *, add0=None, add1
     return _row_norm(x, gamma, beta, add0, add1, int(mode), float(eps), int(dim_actual))
 
 
+# ---------------------------------------------------------------------------
+# projection of a few rows
+# ---------------------------------------------------------------------------
+@custom_op("mia::skinny_linear", mutates_args=())
+def _skinny_linear(x: Tensor, w: Tensor, norm: bool, gamma: Optional[Tensor], eps: float,
+                   dim_actual: int) -> Tensor:
+    return K.skinny_linear(x, w, norm, gamma, eps, dim_actual)
+
+
+@_skinny_linear.register_fake
+def _(x, w, norm, gamma, eps, dim_actual):
+    return x.new_empty((x.shape[0], w.shape[1]))
+
+
+def skinny_linear_ok(x: Tensor, w: Tensor) -> bool:
+    """Shapes and strides the kernel takes, and no gradient wanted (it has
+    none; the library product does)."""
+    return K.skinny_linear_ok(x, w) and not (
+        torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))
+
+
+def skinny_linear(x, w, norm: bool = False, gamma=None, eps: float = 0.0,
+                  dim_actual: int = 0) -> Tensor:
+    if _plain(x, w, gamma):
+        return K.skinny_linear(x, w, bool(norm), gamma, float(eps), int(dim_actual))
+    return _skinny_linear(x, w, bool(norm), gamma, float(eps), int(dim_actual))
+
+
 OPS: List[str] = [
     "kv_write", "gather_kv", "packed_k_convert", "scatter_rows", "stage_rows", "decode_mask",
     "slot_mapping", "remap_null_block", "swa_trim", "paged_decode", "paged_decode_write",
     "paged_prefill",
-    "qkv_epilogue", "row_norm",
+    "qkv_epilogue", "row_norm", "skinny_linear",
 ]
