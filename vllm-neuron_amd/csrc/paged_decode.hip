@@ -1014,33 +1014,55 @@ MIA_DEV void split_body(const P &c) {
       // (qcol, kg) holds q of d = 32 ks + 8 kg + e and O^T of d = 16 blk +
       // 4 kg + i; the dot products are reduced over the 4 lane groups.
       // this wave's run: (o, m, l) into its V buffer (free after the last
-      // tile) and s_one_*; the first wave merges the four runs
+      // tile; 16-byte chunks XOR-swizzled by column, or the 16 columns of a
+      // wave's access share one chunk's banks) and s_one_*; then wave w
+      // merges the runs for d = 16 w .. 16 w + 15.  One wave that merged every
+      // d from unswizzled runs and loaded the active rows 2 bytes at a time
+      // made the 128-token window layer (64 q / 8 kv heads, batch 32) 10.0 us
+      // per layer of a captured step; 8.5 like this, 7.0 against 8.6 at batch 4.
+      static_assert(NW >= DB16, "one merging wave per 16 values of d");
       typedef __attribute__((address_space(3))) f32x4_t lds_f32x4_t;
 #pragma unroll
       for (int blk = 0; blk < DB16; ++blk)
-        *(lds_f32x4_t *)(vw + (qcol * D + 16 * blk + 4 * kg) * 4) = oacc[blk];
+        *(lds_f32x4_t *)(vw + qcol * D * 4 + (((4 * blk + kg) ^ qcol) << 4)) = oacc[blk];
       if (kg == 0) {
         s_one_m[wave][qcol] = m_run;
         s_one_l[wave][qcol] = l_run;
       }
       // the first active token's K/V rows and the sink, loaded by the
-      // merging wave before the barrier (their latency overlaps the other
+      // merging waves before the barrier (their latency overlaps the other
       // waves' runs instead of following the merge)
       const int hq = cur.h * p.G + g_q;
       const int64_t kb0 = cur.b * c.kn_b + (int64_t)cur.h * c.kn_h;
       const int64_t vb0 = cur.b * c.vn_b + (int64_t)cur.h * c.vn_h;
-      uint16_t k0[KSTEPS][8], v0[DB16][4];
+      const int md = 16 * wave + 4 * kg;  // this lane's 4 values of d in the merge
+      u32x4_t k0[KSTEPS];  // 8 bf16 each
+      u32x2_t v0 = {0u, 0u};
       float sink_v = 0.f, vdeq = 1.0f;
-      if (wave == 0) {
+      if (wave < DB16) {
         if (c.v_deq) vdeq = c.v_deq[cur.h];
+        if ((((uintptr_t)c.k_new | (uint64_t)(c.kn_b | c.kn_h) * 2u) & 15u) == 0) {
 #pragma unroll
-        for (int ks = 0; ks < KSTEPS; ++ks)
+          for (int ks = 0; ks < KSTEPS; ++ks)
+            k0[ks] = *reinterpret_cast<const u32x4_t *>(c.k_new + kb0 + kd0(ks, kg));
+        } else {
 #pragma unroll
-          for (int e = 0; e < 8; ++e) k0[ks][e] = c.k_new[kb0 + kd0(ks, kg) + e];
+          for (int ks = 0; ks < KSTEPS; ++ks)
 #pragma unroll
-        for (int blk = 0; blk < DB16; ++blk)
+            for (int e = 0; e < 4; ++e) {
+              const uint16_t *kp = c.k_new + kb0 + kd0(ks, kg) + 2 * e;
+              k0[ks][e] = kp[0] | ((uint32_t)kp[1] << 16);
+            }
+        }
+        if ((((uintptr_t)c.v_new | (uint64_t)(c.vn_b | c.vn_h) * 2u) & 7u) == 0) {
+          v0 = *reinterpret_cast<const u32x2_t *>(c.v_new + vb0 + md);
+        } else {
 #pragma unroll
-          for (int i = 0; i < 4; ++i) v0[blk][i] = c.v_new[vb0 + 16 * blk + 4 * kg + i];
+          for (int e = 0; e < 2; ++e) {
+            const uint16_t *vp = c.v_new + vb0 + md + 2 * e;
+            v0[e] = vp[0] | ((uint32_t)vp[1] << 16);
+          }
+        }
         if (c.sink) sink_v = c.sink[hq];
       }
       // private write slots: the row's cache write, by the last wave (its
@@ -1048,49 +1070,41 @@ MIA_DEV void split_body(const P &c) {
       // of them are masked
       if (c.onepass_write && wave == NW - 1) write_active_rows<D>(c, cur.b, cur.h, lane);
       __syncthreads();
-      if (wave != 0) return;
+      if (wave >= DB16) return;
       float m = -INFINITY, l = 0.f;
 #pragma unroll
       for (int w = 0; w < NW; ++w) m = fmaxf(m, s_one_m[w][qcol]);
+      f32x4_t om = {0.f, 0.f, 0.f, 0.f};
       {
         const float mu = (m == -INFINITY) ? 0.f : m;
-#pragma unroll
-        for (int blk = 0; blk < DB16; ++blk) oacc[blk] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int w = 0; w < NW; ++w) {
           const float f = __builtin_amdgcn_exp2f(s_one_m[w][qcol] - mu);
           l += s_one_l[w][qcol] * f;
           const lds_u8_t *vwo = (lds_u8_t *)&v_lds[w][0];
+          const f32x4_t o =
+              *(const lds_f32x4_t *)(vwo + qcol * D * 4 + (((4 * wave + kg) ^ qcol) << 4));
 #pragma unroll
-          for (int blk = 0; blk < DB16; ++blk) {
-            const f32x4_t o = *(const lds_f32x4_t *)(vwo + (qcol * D + 16 * blk + 4 * kg) * 4);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) oacc[blk][i] += o[i] * f;
-          }
+          for (int i = 0; i < 4; ++i) om[i] += o[i] * f;
         }
       }
       const float vsc = FP8 ? 256.0f : 1.0f;  // cache V was widened x 2^-8
 #pragma unroll
-      for (int blk = 0; blk < DB16; ++blk)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) oacc[blk][i] *= vsc;
-      auto absorb = [&](float sk, const float (&vv)[DB16][4], bool has_v) {
+      for (int i = 0; i < 4; ++i) om[i] *= vsc;
+      auto absorb = [&](float sk, const float (&vv)[4], bool has_v) {
         const float m_new = fmaxf(m, sk);
         const float mu = (m_new == -INFINITY) ? 0.f : m_new;
         const float a = __builtin_amdgcn_exp2f(m - mu);
         const float pk = __builtin_amdgcn_exp2f(sk - mu);
         l = l * a + pk;
 #pragma unroll
-        for (int blk = 0; blk < DB16; ++blk)
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            oacc[blk][i] = oacc[blk][i] * a + (has_v ? pk * vv[blk][i] : 0.f);
+        for (int i = 0; i < 4; ++i) om[i] = om[i] * a + (has_v ? pk * vv[i] : 0.f);
         m = m_new;
       };
       const float ascale = c.act_scale_log2 * kdq_cur;
       // active token k with its K and V rows as floats (after the cache's
       // quantise round trip)
-      auto active_token = [&](int k, const float (&kf)[KSTEPS][8], const float (&vf)[DB16][4]) {
+      auto active_token = [&](int k, const float (&kf)[KSTEPS][8], const float (&vf)[4]) {
         float dot = 0.f;
 #pragma unroll
         for (int ks = 0; ks < KSTEPS; ++ks) {
@@ -1120,27 +1134,24 @@ MIA_DEV void split_body(const P &c) {
       // general form, with the round trip inlined for every element, made
       // this tail ~5k instructions that the wave fetched past.
       if (p.S > 0) {
-        float kf[KSTEPS][8], vf[DB16][4];
+        float kf[KSTEPS][8], vf[4];
+        auto k0f = [&](int ks, int e) { return (e & 1) ? bf16hi(k0[ks][e >> 1]) : bf16lo(k0[ks][e >> 1]); };
+        auto v0f = [&](int i) { return (i & 1) ? bf16hi(v0[i >> 1]) : bf16lo(v0[i >> 1]); };
         if (__builtin_expect(c.quant_mode == MIA_QUANT_NONE, 1)) {
 #pragma unroll
           for (int ks = 0; ks < KSTEPS; ++ks)
 #pragma unroll
-            for (int e = 0; e < 8; ++e) kf[ks][e] = bf16_bits_to_f32(k0[ks][e]);
+            for (int e = 0; e < 8; ++e) kf[ks][e] = k0f(ks, e);
 #pragma unroll
-          for (int blk = 0; blk < DB16; ++blk)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) vf[blk][i] = bf16_bits_to_f32(v0[blk][i]);
+          for (int i = 0; i < 4; ++i) vf[i] = v0f(i);
         } else {
 #pragma unroll
           for (int ks = 0; ks < KSTEPS; ++ks)
 #pragma unroll
             for (int e = 0; e < 8; ++e)
-              kf[ks][e] = quant_roundtrip(c, bf16_bits_to_f32(k0[ks][e]), cur.h, c.k_quant);
+              kf[ks][e] = quant_roundtrip(c, k0f(ks, e), cur.h, c.k_quant);
 #pragma unroll
-          for (int blk = 0; blk < DB16; ++blk)
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-              vf[blk][i] = quant_roundtrip(c, bf16_bits_to_f32(v0[blk][i]), cur.h, c.v_quant);
+          for (int i = 0; i < 4; ++i) vf[i] = quant_roundtrip(c, v0f(i), cur.h, c.v_quant);
         }
         active_token(0, kf, vf);
       }
@@ -1148,7 +1159,7 @@ MIA_DEV void split_body(const P &c) {
       for (int k = 1; __builtin_expect(k < p.S, 0); ++k) {
         const int64_t kb = cur.b * c.kn_b + (int64_t)k * c.kn_s + (int64_t)cur.h * c.kn_h;
         const int64_t vb = cur.b * c.vn_b + (int64_t)k * c.vn_s + (int64_t)cur.h * c.vn_h;
-        float kf[KSTEPS][8], vf[DB16][4];
+        float kf[KSTEPS][8], vf[4];
 #pragma unroll
         for (int ks = 0; ks < KSTEPS; ++ks)
 #pragma unroll
@@ -1156,15 +1167,12 @@ MIA_DEV void split_body(const P &c) {
             kf[ks][e] = quant_roundtrip(c, bf16_bits_to_f32(c.k_new[kb + kd0(ks, kg) + e]), cur.h,
                                         c.k_quant);
 #pragma unroll
-        for (int blk = 0; blk < DB16; ++blk)
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            vf[blk][i] = quant_roundtrip(c, bf16_bits_to_f32(c.v_new[vb + 16 * blk + 4 * kg + i]),
-                                         cur.h, c.v_quant);
+        for (int i = 0; i < 4; ++i)
+          vf[i] = quant_roundtrip(c, bf16_bits_to_f32(c.v_new[vb + md + i]), cur.h, c.v_quant);
         active_token(k, kf, vf);
       }
       if (c.sink) {  // the sink logit joins the denominator only
-        const float vz[DB16][4] = {};
+        const float vz[4] = {};
         absorb(sink_v * kLog2e, vz, false);
       }
       if (col_ok) {
@@ -1173,19 +1181,14 @@ MIA_DEV void split_body(const P &c) {
         // when the output allows it
         const bool st8 = (((uintptr_t)c.out | (uint64_t)(c.os_b | c.os_s | c.os_h) * 2u) & 7u) == 0;
         const float inv = vdeq / l;  // one division instead of one per element
+        const u32x2_t o4 = {pack2_bf16(om[0] * inv, om[1] * inv),
+                            pack2_bf16(om[2] * inv, om[3] * inv)};
+        uint16_t *dst = op + md;
+        if (st8) {
+          *reinterpret_cast<u32x2_t *>(dst) = o4;
+        } else {
 #pragma unroll
-        for (int blk = 0; blk < DB16; ++blk) {
-          uint16_t o4[4];
-#pragma unroll
-          for (int i = 0; i < 4; ++i) o4[i] = (uint16_t)f32_to_bf16_bits(oacc[blk][i] * inv);
-          uint16_t *dst = op + 16 * blk + 4 * kg;
-          if (st8) {
-            *reinterpret_cast<u32x2_t *>(dst) =
-                u32x2_t{o4[0] | ((uint32_t)o4[1] << 16), o4[2] | ((uint32_t)o4[3] << 16)};
-          } else {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) dst[i] = o4[i];
-          }
+          for (int i = 0; i < 4; ++i) dst[i] = (uint16_t)(o4[i >> 1] >> (16 * (i & 1)));
         }
       }
       break;
