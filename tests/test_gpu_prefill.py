@@ -447,3 +447,33 @@ def test_single_sequence_even_split(gpu, case):
                          None if sink is None else sink.cpu())
     err = (got[first:].float().cpu().double() - f).abs().max().item()
     assert err <= (TOL_FP8 if fp8 else TOL_BF16), err
+
+
+def test_single_sequence_without_workspace(gpu):
+    """The C entry with no workspace runs a short single sequence unsplit
+    (the wrapper would allocate one for the even split)."""
+    import ctypes
+
+    from vllm_neuron_amd import _native as N
+
+    cfg = W.PrefillConfig("t", 1, 8, 2, 128, 32, 64, 2048, 2048, seed=7)
+    b = W.make_prefill_batch(cfg, gpu)
+    K.kv_write(b.k_new, b.v_new, b.slots, b.k_cache, b.v_cache)
+    base = K.paged_prefill(b.q, b.cu_seqlens, b.prior, 64, b.k_cache, b.v_cache, b.block_table,
+                           scale=0.1, split_tokens=1 << 20)
+    out = torch.zeros_like(base)
+    a = N.PrefillArgs()
+    a.q, a.q_stride = b.q.data_ptr(), tuple(b.q.stride())
+    a.num_seqs, a.max_seqlen_q, a.num_tokens = 1, 64, 64
+    a.cu_seqlens_q, a.prior_tokens = b.cu_seqlens.data_ptr(), b.prior.data_ptr()
+    a.k_cache, a.v_cache = b.k_cache.data_ptr(), b.v_cache.data_ptr()
+    a.cache_dtype = a.out_dtype = N.DTYPE_BF16
+    a.k_cache_stride, a.v_cache_stride = (*b.k_cache.stride(), 0), tuple(b.v_cache.stride())
+    a.num_blocks, a.block_size = b.k_cache.shape[0], 32
+    a.block_table, a.blocks_per_seq = b.block_table.data_ptr(), b.block_table.shape[1]
+    a.bt_stride = (b.block_table.stride(0), 0, 1)
+    a.num_q_heads, a.num_kv_heads, a.head_dim, a.scale = 8, 2, 128, 0.1
+    a.out, a.out_stride = out.data_ptr(), tuple(out.stride())
+    assert N.lib().mia_prefill_workspace_bytes(ctypes.byref(a)) > 0
+    N.check(N.lib().mia_paged_prefill(ctypes.byref(a), N.stream_ptr(gpu)), "paged_prefill")
+    assert torch.equal(out, base)

@@ -389,7 +389,11 @@ int mia_paged_prefill(const mia_prefill_args *a, mia_stream_t stream) {
   if (a->num_seqs == 0) return MIA_OK;
   int rc = validate_prefill(a);
   if (rc) return rc;
-  const mia::PrefillPlan pl = mia::plan_prefill(*a);
+  mia::PrefillPlan pl = mia::plan_prefill(*a);
+  // a caller that passes no (or a smaller) workspace keeps the launch that
+  // needs none where there is one
+  if (pl.even && pl.ws_bytes > 0 && (!a->workspace || a->workspace_bytes < pl.ws_bytes))
+    pl = mia::plan_prefill(*a, false);
   if (pl.ws_bytes > 0) {
     MIA_REQUIRE(a->workspace && a->workspace_bytes >= pl.ws_bytes, MIA_ERR_VALUE,
                 "prefill: workspace too small (query mia_prefill_workspace_bytes)");

@@ -74,7 +74,8 @@ struct PrefillPlan {
   int slots;         // workgroups resident on the device at once
   size_t ws_bytes;   // workspace bytes (0 without split)
 };
-PrefillPlan plan_prefill(const mia_prefill_args &a);
+// even = false: without the even split of a single sequence (and its workspace).
+PrefillPlan plan_prefill(const mia_prefill_args &a, bool even = true);
 int launch_paged_prefill(const mia_prefill_args &a, const PrefillPlan &p, hipStream_t s);
 
 }  // namespace mia

@@ -537,7 +537,8 @@ struct RowMax {
 MIA_DEV float exp_tile(const f32x16_t (&sacc)[2], uint32_t (&pk)[2][8]) {
   typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
   const bf16x2_t ones = {(__bf16)1.0f, (__bf16)1.0f};
-  float psum = 0.f;
+  // four chains of adds: the test of the sum waits for their end
+  float psum[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
@@ -545,10 +546,11 @@ MIA_DEV float exp_tile(const f32x16_t (&sacc)[2], uint32_t (&pk)[2][8]) {
       const float p0 = __builtin_amdgcn_exp2f(sacc[kb][e]);
       const float p1 = __builtin_amdgcn_exp2f(sacc[kb][e + 1]);
       pk[kb][e >> 1] = pack2_bf16(p0, p1);
-      psum = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, pk[kb][e >> 1]), ones,
-                                             psum, false);
+      float &s = psum[2 * kb + ((e >> 1) & 1)];
+      s = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, pk[kb][e >> 1]), ones, s,
+                                          false);
     }
-  return psum;
+  return (psum[0] + psum[1]) + (psum[2] + psum[3]);
 }
 
 // max over the two lanes l and l ^ 32 of a row (its two key groups)
@@ -937,7 +939,9 @@ static_assert(waitcnt_vm(4) == 0xF74 && waitcnt_vm(0) == 0xF70, "vmcnt encoding"
 // d = 80, not causal (86 GFLOP of useful channels): 133 us with all 128 channels,
 // 112 with 80; the call, which also no longer stages q, 141 -> 113.
 // Reading fragments ahead, as at d = 64, measured 2 % slower.
-template <int D, int WAVES, int STAGES, bool FP8, bool PK, int DU = D>
+// NARROW: q and out rows hold d_used < D channels; the full-width kernels test
+// nothing (the tests cost the mixed batch 0.7 %).
+template <int D, int WAVES, int STAGES, bool FP8, bool PK, int DU = D, bool NARROW = DU != D>
 __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void prefill_dma_kernel(
     PrefillKParams p) {
   static_assert(DU == D || (D == 128 && !FP8 && DU > 64 && DU % 16 == 0), "padded head dims");
@@ -1056,7 +1060,7 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void prefill_dma_kernel(
                          (int64_t)(row_ok ? hq : 0) * p.qs_h;
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ++ks)
-      qw[ks] = ks * 16 + half * 8 < p.d_used
+      qw[ks] = !NARROW || ks * 16 + half * 8 < p.d_used
                    ? *reinterpret_cast<const u32x4_t *>(qp + ks * 16 + half * 8)
                    : u32x4_t{0u, 0u, 0u, 0u};
   }
@@ -1413,7 +1417,7 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void prefill_dma_kernel(
             ob + rl2 * ROWB + ((ch ^ (rl2 & (CH - 1))) << 4));
         const int r2 = row0 + wave * kRowsW + rl2;
         if (r2 < rows_total && q_begin + r2 / G < p.num_tokens &&
-            pass * (D / 2) + ch * 4 < p.d_used)
+            (!NARROW || pass * (D / 2) + ch * 4 < p.d_used))
           *reinterpret_cast<f32x4_t *>(part + first + rl2 * step + pass * (D / 2) + ch * 4) = v;
       }
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // read before the next pass writes
@@ -1446,7 +1450,8 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void prefill_dma_kernel(
         ob + rl2 * ROWB + ((ch ^ (rl2 & (CH - 1))) << 4));
     const int r2 = row0 + wave * kRowsW + rl2;
     const int pos2 = r2 / G;
-    if (r2 >= rows_total || q_begin + pos2 >= p.num_tokens || ch * 8 >= p.d_used) continue;
+    if (r2 >= rows_total || q_begin + pos2 >= p.num_tokens || (NARROW && ch * 8 >= p.d_used))
+      continue;
     if (split) {
       uint8_t *w = p.ws + ((((int64_t)seq * p.Hkv + h) * p.rows_max + r2) * p.nsplit + sp) *
                               (int64_t)part_bytes(D);
@@ -1643,6 +1648,8 @@ bool use_dma_kernel(const mia_prefill_args &a) {
   // the copies address K and V with one block offset and one token stride
   // (packed K: the stride of the even token of a pair)
   const int64_t k_tok = a.k_packed ? a.k_cache_stride[2] / 2 : a.k_cache_stride[2];
+  // padded FP8 caches run the register-staged kernel
+  if (a.cache_dtype != MIA_DTYPE_BF16 && prefill_head_dim_used(a) < a.head_dim) return false;
   // d = 64: bf16 caches.  Compact launches and FP8 caches of that head dim
   // keep the register-staged kernel.
   const bool dim_ok = a.head_dim == 128 || (a.cache_dtype == MIA_DTYPE_BF16 && !a.compact_kernel);
@@ -1740,7 +1747,7 @@ void plan_even(const mia_prefill_args &a, bool half_ok, PrefillPlan &pl) {
 
 }  // namespace
 
-PrefillPlan plan_prefill(const mia_prefill_args &a) {
+PrefillPlan plan_prefill(const mia_prefill_args &a, bool even) {
   PrefillPlan pl{};
   // compact: workgroups that fit on a CU beside a decode workgroup (the
   // copy ring with 4 waves and 2 stages, 72 KiB of LDS; FP8 caches and
@@ -1793,7 +1800,7 @@ PrefillPlan plan_prefill(const mia_prefill_args &a) {
     pl.ws_bytes = (size_t)a.num_seqs * a.num_kv_heads * pl.rows_max * pl.nsplit *
                   part_bytes(a.head_dim);
   }
-  if (a.split_tokens <= 0 && a.num_seqs == 1 && !a.compact_kernel && !a.bound_min &&
+  if (even && a.split_tokens <= 0 && a.num_seqs == 1 && !a.compact_kernel && !a.bound_min &&
       pl.rows_max > 0)
     plan_even(a, pl.dma && a.cache_dtype == MIA_DTYPE_BF16 && a.blocks_per_seq <= dma_ids(4), pl);
   return pl;
@@ -1864,12 +1871,21 @@ int launch_paged_prefill(const mia_prefill_args &a, const PrefillPlan &pl, hipSt
                             : dim3((unsigned)((pl.rows_max + pl.rows_wg - 1) / pl.rows_wg),
                                    (unsigned)a.num_kv_heads,
                                    (unsigned)(pl.nsplit * a.num_seqs));
+  const bool narrow = kp.d_used < a.head_dim;
   if (pl.dma && a.head_dim == 64 && pl.dma_waves == 4) {
-    hipLaunchKernelGGL((prefill_dma_kernel<64, 4, kDmaStages, false, false>), grid, dim3(4 * 64),
-                       0, s, kp);
+    if (narrow)
+      hipLaunchKernelGGL((prefill_dma_kernel<64, 4, kDmaStages, false, false, 64, true>), grid,
+                         dim3(4 * 64), 0, s, kp);
+    else
+      hipLaunchKernelGGL((prefill_dma_kernel<64, 4, kDmaStages, false, false>), grid, dim3(4 * 64),
+                         0, s, kp);
   } else if (pl.dma && a.head_dim == 64) {
-    hipLaunchKernelGGL((prefill_dma_kernel<64, kDmaWaves, kDmaStages, false, false>), grid,
-                       dim3(kDmaWaves * 64), 0, s, kp);
+    if (narrow)
+      hipLaunchKernelGGL((prefill_dma_kernel<64, kDmaWaves, kDmaStages, false, false, 64, true>),
+                         grid, dim3(kDmaWaves * 64), 0, s, kp);
+    else
+      hipLaunchKernelGGL((prefill_dma_kernel<64, kDmaWaves, kDmaStages, false, false>), grid,
+                         dim3(kDmaWaves * 64), 0, s, kp);
   } else if (pl.dma && pl.dma_waves == 4) {
     if (kp.d_used <= 80)
       hipLaunchKernelGGL((prefill_dma_kernel<128, 4, 2, false, false, 80>), grid, dim3(4 * 64), 0,
@@ -1877,6 +1893,9 @@ int launch_paged_prefill(const mia_prefill_args &a, const PrefillPlan &pl, hipSt
     else if (kp.d_used <= 96)
       hipLaunchKernelGGL((prefill_dma_kernel<128, 4, 2, false, false, 96>), grid, dim3(4 * 64), 0,
                          s, kp);
+    else if (narrow)
+      hipLaunchKernelGGL((prefill_dma_kernel<128, 4, 2, false, false, 128, true>), grid,
+                         dim3(4 * 64), 0, s, kp);
     else
       hipLaunchKernelGGL((prefill_dma_kernel<128, 4, 2, false, false>), grid, dim3(4 * 64), 0, s,
                          kp);
@@ -1893,6 +1912,10 @@ int launch_paged_prefill(const mia_prefill_args &a, const PrefillPlan &pl, hipSt
     else if (kp.d_used <= 96)
       hipLaunchKernelGGL((prefill_dma_kernel<128, kDmaWaves, kDmaStages, false, false, 96>), grid,
                          dim3(kDmaWaves * 64), 0, s, kp);
+    else if (narrow)
+      hipLaunchKernelGGL(
+          (prefill_dma_kernel<128, kDmaWaves, kDmaStages, false, false, 128, true>), grid,
+          dim3(kDmaWaves * 64), 0, s, kp);
     else
       hipLaunchKernelGGL((prefill_dma_kernel<128, kDmaWaves, kDmaStages, false, false>), grid,
                          dim3(kDmaWaves * 64), 0, s, kp);
