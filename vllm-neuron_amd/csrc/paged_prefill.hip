@@ -960,6 +960,11 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void prefill_dma_kernel(
   constexpr int CH = ROWB / 16;        // 16-byte chunks per row
   constexpr int RPI = 64 / CH;         // rows per DMA instruction
   constexpr bool AHEAD = D == 64;      // LDS operands read ahead of the products
+  // key steps of V^T read before the softmax: with one wave per SIMD (4 waves)
+  // the first covers part of the LDS latency (777 tokens after 1536: 53.5 ->
+  // 52.7 us, the mixed batch's compact launch 0.4 %; two steps or K ahead: no
+  // further gain)
+  constexpr int VPRE = AHEAD ? 4 : WAVES == 4 ? 1 : 0;
   constexpr int EB = FP8 ? 1 : 2;      // cache bytes per element
   constexpr int TILE8 = kKT * D;       // bytes per FP8 K (or V) tile
   constexpr int NJ8 = 8 / kDmaWaves;   // FP8 DMA instructions per thread per tile
@@ -1199,10 +1204,10 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void prefill_dma_kernel(
       return u32x4_t{__builtin_bit_cast(u32x2_t, t2[0])[0], __builtin_bit_cast(u32x2_t, t2[0])[1],
                      __builtin_bit_cast(u32x2_t, t2[1])[0], __builtin_bit_cast(u32x2_t, t2[1])[1]};
     };
-    u32x4_t vf[AHEAD ? 4 : 1][DBLK];
-    if constexpr (AHEAD) {  // the softmax covers the reads of V^T
+    u32x4_t vf[VPRE > 0 ? VPRE : 1][DBLK];
+    if constexpr (VPRE > 0) {  // the softmax covers these reads
 #pragma unroll
-      for (int ks2 = 0; ks2 < 4; ++ks2)
+      for (int ks2 = 0; ks2 < VPRE; ++ks2)
 #pragma unroll
         for (int db = 0; db < DBLK; ++db) vf[ks2][db] = read_v(ks2, db);
       __builtin_amdgcn_sched_barrier(0);
@@ -1219,9 +1224,9 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void prefill_dma_kernel(
       const bf16x8_t bop = __builtin_bit_cast(bf16x8_t, bw);
 #pragma unroll
       for (int db = 0; db < DBLK; ++db) {
-        if constexpr (!AHEAD) vf[0][db] = read_v(ks2, db);
+        const u32x4_t v = ks2 < VPRE ? vf[ks2 < VPRE ? ks2 : 0][db] : read_v(ks2, db);
         acc_o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-            __builtin_bit_cast(bf16x8_t, vf[AHEAD ? ks2 : 0][db]), bop, acc_o[db], 0, 0, 0);
+            __builtin_bit_cast(bf16x8_t, v), bop, acc_o[db], 0, 0, 0);
       }
     }
   };
