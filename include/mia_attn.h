@@ -332,10 +332,11 @@ typedef struct {
   /* Split-K over keys: a long sequence's keys are cut into chunks of
    * split_tokens (a multiple of 64; 0 = chosen from the shapes) processed by
    * separate workgroups, whose partials (bf16 o, fp32 max and sum) go to
-   * `workspace` and are
-   * merged by a second kernel.  workspace_bytes must be at least
-   * mia_prefill_workspace_bytes(args) (0 when no split is planned; then
-   * workspace may be NULL). */
+   * `workspace` and are merged by a second kernel.  With split_tokens 0 the row
+   * tiles of one sequence may instead be cut evenly on the device (fp32 o); a
+   * call without the workspace for that runs as if it were not.
+   * workspace_bytes must be at least mia_prefill_workspace_bytes(args) (0 when
+   * no split is planned; then workspace may be NULL). */
   void *workspace;
   size_t workspace_bytes;
   int32_t split_tokens;

@@ -6,9 +6,11 @@ validation and error classes (:1484-1575, :1724-1741), the block-KV cache
 layout and the output layouts (:1163-1182).
 
 What runs where
-  * Stage 1 (input RMS norm) is the HIP row norm ``mia_row_norm``; stages 2
-    and 9 (QKV and output projections) are library GEMMs (bf16 inputs,
-    fp32 accumulation, bias fused); stages 3-6.5 (head split, QK RMS norm
+  * Up to 16 rows without a bias, stages 1 and 2 (input RMS norm, QKV
+    projection) are one HIP launch, ``mia_skinny_linear``, and stage 9 (output
+    projection) another; otherwise stage 1 is the HIP row norm
+    ``mia_row_norm`` and stages 2 and 9 are library GEMMs (bf16 inputs, fp32
+    accumulation, bias fused); stages 3-6.5 (head split, QK RMS norm
     before / after RoPE, RoPE in the half-split or interleaved layout, with
     the reference's bf16 rounding of each RoPE product and sum) are one
     HIP epilogue pass ``mia_qkv_epilogue``.
