@@ -518,3 +518,18 @@ def test_decode_block_few_rows_equal_many(gpu):
                                      pos_ids=pos[:n].contiguous(), **kw)[0])
     a, b = outs[0][:4].double(), outs[1].double()
     assert (a - b).abs().max().item() <= 2e-2 * max(1.0, a.abs().max().item())
+
+
+def test_skinny_linear_gamma_forms(gpu):
+    """gamma on the host, unaligned or strided gives the same bits as the
+    aligned bf16 vector on the device."""
+    g = torch.Generator().manual_seed(3)
+    x = torch.randn(4, 256, generator=g).to(bf).to(gpu)
+    w = torch.randn(256, 64, generator=g).to(bf).to(gpu)
+    gam = (torch.rand(256, generator=g) + 0.5).to(bf)
+    wide = torch.zeros(512, dtype=bf)
+    wide[1::2] = gam
+    base = K.skinny_linear(x, w, True, gam.to(gpu), 1e-5)
+    off = torch.cat([gam[:1], gam]).to(gpu)[1:]
+    for form in (gam, off, wide.to(gpu)[1::2], gam.float().to(gpu)):
+        assert torch.equal(K.skinny_linear(x, w, True, form, 1e-5), base)

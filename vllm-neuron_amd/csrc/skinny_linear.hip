@@ -24,7 +24,7 @@
 // -> 24.9, 2880 x 5120 28.8 -> 21.3, 8192 x 4096 48.6 -> 42.6; without the norm
 // 2048 x 2048 8.8 -> 7.2, 4096 x 4096 21.9 -> 19.0.  64 columns per workgroup
 // (whole lines, half the workgroups): 2048 x 3072 with norm 11.7; nontemporal
-// weight loads 13.8.  From N = 8192 on (more than one workgroup per CU) the
+// weight loads 13.8.  Past N = 8192 (more than one workgroup per CU) the
 // library is faster: 8192 x 10240 53.8 against 89.9.
 #include "mia_device.h"
 #include "mia_internal.h"

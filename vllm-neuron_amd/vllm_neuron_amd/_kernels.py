@@ -959,7 +959,7 @@ def skinny_linear(x: torch.Tensor, w: torch.Tensor, norm: bool = False,
     """``x [T, K] @ w [K, N]`` for T <= 16 (``skinny_linear_ok``), with
     ``norm`` of the RMS-normalised rows (``row_norm`` mode 1).  Rows whose
     address is not vector aligned are copied first."""
-    dev = N.require_gpu(x, w, gamma)
+    dev = N.require_gpu(x, w)
     if not skinny_linear_ok(x, w):
         raise NotImplementedError("skinny_linear: unsupported shapes, strides or dtypes")
     if x.data_ptr() % 16:
@@ -981,8 +981,8 @@ def skinny_linear(x: torch.Tensor, w: torch.Tensor, norm: bool = False,
         if gamma is not None:
             if gamma.numel() < k:
                 raise ValueError(f"gamma has {gamma.numel()} entries, needs {k}")
-            if not (gamma.dtype == torch.bfloat16 and gamma.is_contiguous()
-                    and gamma.data_ptr() % 16 == 0):
+            if not (gamma.dtype == torch.bfloat16 and gamma.device == dev
+                    and gamma.is_contiguous() and gamma.data_ptr() % 16 == 0):
                 gamma = _scale_f32(gamma, dev, k, "gamma")
             a.gamma = gamma.data_ptr()
             a.gamma_bf16 = 1 if gamma.dtype == torch.bfloat16 else 0
