@@ -477,3 +477,51 @@ def test_single_sequence_without_workspace(gpu):
     assert N.lib().mia_prefill_workspace_bytes(ctypes.byref(a)) > 0
     N.check(N.lib().mia_paged_prefill(ctypes.byref(a), N.stream_ptr(gpu)), "paged_prefill")
     assert torch.equal(out, base)
+
+
+def _cache_of(rows, bs, dtype, gpu, packed=False):
+    """Block cache ``[1 + n / bs, 1, bs, d]`` (null block 0) and table of one
+    sequence from its rows ``[n, d]``."""
+    n, d = rows.shape
+    c = torch.zeros(1 + n // bs, 1, bs, d)
+    c[1:, 0] = rows.view(n // bs, bs, d)
+    return c.to(dtype).to(gpu), torch.arange(1, 1 + n // bs, dtype=torch.int32, device=gpu)[None]
+
+
+@pytest.mark.parametrize("d, bs, dtype, compact", [
+    (64, 32, torch.bfloat16, False),   # copy ring
+    (64, 4, torch.bfloat16, False),    # register-staged
+    (128, 32, torch.bfloat16, False),  # copy ring
+    (128, 32, torch.bfloat16, True),   # four waves, tested by the maximum
+    (128, 4, torch.bfloat16, False),
+    (128, 32, torch.float8_e4m3fn, False),
+    (64, 32, torch.float8_e4m3fn, False),
+])
+def test_maximum_moves_past_8_only(gpu, d, bs, dtype, compact):
+    """The running maximum moves when a score passes it by more than 8 (log2
+    units), whatever the tile's sum is: one key of score 0, then 64 keys of
+    score 5.34375 whose V is 0.  Their weights 2^5.34375 = 40.61 are rounded to
+    bf16 (40.5), so a channel of the first key's V comes out as v / (1 + 64 *
+    40.5); a maximum moved to 5.34375 would give v / (1 + 64 * 40.61)."""
+    n = 128
+    k = torch.zeros(n, d)
+    k[1:64, 2] = -192.0  # no weight
+    k[64:, 0], k[64:, 1] = 5.0, 0.34375
+    v = torch.zeros(n, d)
+    ch = torch.arange(d)
+    v[0] = (8 + ch % 8) / 8.0 * 2.0 ** (ch // 8 % 4)
+    kc, table = _cache_of(k, bs, dtype, gpu)
+    vc, _ = _cache_of(v, bs, dtype, gpu)
+    q = torch.zeros(1, 1, d, dtype=torch.bfloat16, device=gpu)
+    q[0, 0, :3] = 1.0
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=gpu)
+    out = K.paged_prefill(q, i32([0, 1]), i32([n - 1]), 1, kc, vc, table,
+                          scale=0.6931471805599453, compact_kernel=compact)
+    got = out[0, 0].double().cpu()
+    want = (v[0].double() / (1 + 64 * 40.5))
+    moved = (v[0].double() / (1 + 64 * 2.0 ** 5.34375)).to(torch.bfloat16).double()
+    # half a bf16 step is 2^-9 relative at most; the fp32 steps add some 2^-22
+    assert bool(((got - want).abs() <= want * (2.0 ** -8)).all())
+    bits = want.to(torch.bfloat16).double()
+    assert int((bits != moved).sum()) >= d // 8  # the two rules are told apart
+    assert torch.equal(got, bits)
