@@ -525,3 +525,56 @@ def test_maximum_moves_past_8_only(gpu, d, bs, dtype, compact):
     bits = want.to(torch.bfloat16).double()
     assert int((bits != moved).sum()) >= d // 8  # the two rules are told apart
     assert torch.equal(got, bits)
+
+
+@pytest.mark.parametrize("Hq, Hkv, d, bs, fp8, packed, new, prior, window, compact", [
+    (8, 2, 64, 32, False, False, 100, 41, 0, False),     # copy ring: keys end inside a block
+    (8, 2, 64, 16, False, False, 70, 129, 0, False),     # and a table entry of -1 inside the tile
+    (8, 2, 64, 16, False, False, 200, 1000, 128, False),  # freed blocks before the window
+    (8, 2, 64, 4, False, False, 100, 41, 50, False),     # register-staged
+    (8, 2, 64, 32, False, False, 65, 5000, 0, False),    # chunks of an even split
+    (8, 2, 128, 32, False, False, 100, 41, 0, False),
+    (8, 2, 128, 16, False, False, 200, 1000, 128, False),
+    (8, 2, 128, 32, False, False, 300, 500, 0, True),    # two-stage ring
+    (8, 2, 128, 128, False, False, 1, 0, 0, False),      # a single key
+    (8, 2, 128, 64, True, False, 100, 41, 0, False),
+    (8, 2, 128, 64, True, True, 90, 1000, 128, False),
+    (8, 2, 64, 32, True, False, 100, 41, 33, False),
+])
+def test_unattended_cache_slots_do_not_matter(gpu, Hq, Hkv, d, bs, fp8, packed, new, prior, window,
+                                              compact):
+    """Slots that no row sees (past the last key, of the null block, of blocks
+    freed before the window) may hold NaN: the outputs are those over a cache
+    that holds zeros there, bit for bit."""
+    g = torch.Generator().manual_seed(91)
+    n = prior + new
+    used = -(-n // bs)
+    first = max(0, prior - window + 1) // bs if window else 0  # blocks before it are freed
+    table = torch.full((1, used + 7), -1, dtype=torch.int32)
+    table[0, :used] = 1 + torch.randperm(used, generator=g).to(torch.int32)
+    table[0, :first] = 0
+    dt = torch.float8_e4m3fn if fp8 else torch.bfloat16
+
+    def cache(rows, fill):
+        c = torch.full((used + 2, Hkv, bs, d), fill)
+        for j in range(first, used):
+            m = min(bs, n - j * bs)
+            c[table[0, j], :, :m] = rows[:, j * bs:j * bs + m]
+        return c.to(dt)
+
+    def pack(c):  # [nb, Hkv, bs, d] -> [nb, Hkv, bs / 2, d, 2]
+        return c.view(torch.uint8).view(*c.shape[:2], bs // 2, 2, d).transpose(3, 4).contiguous().view(dt)
+
+    kr, vr = (torch.randn(Hkv, n, d, generator=g) for _ in range(2))
+    q = torch.randn(new, Hq, d, generator=g).to(torch.bfloat16).to(gpu)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=gpu)
+
+    def run(fill):
+        kc, vc = cache(kr, fill), cache(vr, fill)
+        return K.paged_prefill(q, i32([0, new]), i32([prior]), new, (pack(kc) if packed else kc).to(gpu),
+                               vc.to(gpu), table.to(gpu), scale=d ** -0.5, sliding_window=window,
+                               k_packed=packed, compact_kernel=compact)
+
+    clean, dirty = run(0.0), run(float("nan"))
+    assert torch.isfinite(clean.float()).all()
+    assert torch.equal(clean.view(torch.int16), dirty.view(torch.int16))

@@ -738,8 +738,10 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillKParams p) {
   if (sp >= kr.n_sp) return;  // no chunk for this workgroup
   int kt0, kt_last;
   chunk_tiles(p, kr, ksplit, sp, kt0, kt_last);
-  // clamp a key into [kt0, kmax) so every load hits an attended block
-  auto clampk = [&](int k) { return min(max(k, kt0), max(kmax - 1, kt0)); };
+  // clamp a key to those of the tiles that some row sees: other cache slots
+  // (unwritten, freed or the null block's) may hold NaN, and 0 * NaN is NaN
+  const int k_first = max(kt0, kr.kmin);
+  auto clampk = [&](int k) { return min(max(k, k_first), max(kmax - 1, k_first)); };
   auto phys_of = [&](int key) {
     const uint32_t bi = fdiv((uint32_t)clampk(key), p.bs_div);
     int32_t v = p.bt[bt_row + (int64_t)bi * p.bt_j];
@@ -766,8 +768,9 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillKParams p) {
       }
     }
     {
-      // the 4 keys of a group share a block (block_size % 4 == 0); keys at
-      // or past kmax re-read key kmax-1, which lies in the same block
+      // the 4 keys of a group share a block (block_size % 4 == 0); keys
+      // outside [k_first, kmax) re-read the nearest key inside, which lies in
+      // the same block
       const int key = clampk(kt + vg * 4);
       const int off = key - (int)fdiv((uint32_t)key, p.bs_div) * p.bs;
       const uint8_t *src = p.v_cache + ((int64_t)vphys * p.vc_blk + (int64_t)h * p.vc_h +
@@ -1237,6 +1240,15 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void prefill_dma_kernel(
     }
   };
 
+  // Keys of a tile outside the workgroup's range [kmin, kmax): the copies take
+  // whole tiles, and cache slots that no row sees (unwritten, freed or the
+  // null block's) may hold NaN or Inf.  Their scores are masked, but 0 * V is
+  // NaN there, so their V rows are cleared in LDS: by the threads that widen
+  // them (FP8), or, on the first and last tile alone, between the copy and the
+  // step of the tile (one more barrier).
+  const int kmin = readfirstlane(kr.kmin), kmax = readfirstlane(kr.kmax);
+  auto cut_tile = [&](int kt) { return kt < kmin || kt + kKT > kmax; };
+
   // ---- copy ring of STAGES stages.  At the top of a step this thread waits
   // for its own copies of tile kt (those of the tiles issued after it may
   // stay in flight: 2 * NJ instructions per tile), then the barrier makes
@@ -1276,7 +1288,7 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void prefill_dma_kernel(
       // t / 8, FP8 chunk t % 8 (channels 16c' .. 16c'+15 = bf16 chunks 2c',
       // 2c'+1), written at the swizzled places the products read
       typedef __attribute__((address_space(3))) u32x4_t lds_u32x4_t;
-      auto widen = [&](int stg, int bb) {
+      auto widen = [&](int kt, int stg, int bb) {
         const lds_u8_t8 *s8 = (const lds_u8_t8 *)&kv8_lds[stg][0][0];
         lds_u8_t *kb = kv_base + bb * 2 * TILEB;
         lds_u8_t *vb = kb + TILEB;
@@ -1284,7 +1296,9 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void prefill_dma_kernel(
           const int row = tid >> 3, c8 = tid & 7;
 #pragma unroll
           for (int kv = PK ? 1 : 0; kv < 2; ++kv) {
-            const u32x4_t w = *(const lds_u32x4_t *)(s8 + kv * TILE8 + row * D + (c8 << 4));
+            u32x4_t w = *(const lds_u32x4_t *)(s8 + kv * TILE8 + row * D + (c8 << 4));
+            if (kv == 1 && cut_tile(kt) && (kt + row < kmin || kt + row >= kmax))
+              w = u32x4_t{0u, 0u, 0u, 0u};
             const u32x4_t lo = e4m3fn_x8_to_bf16_scaled(u32x2_t{w[0], w[1]});
             const u32x4_t hi = e4m3fn_x8_to_bf16_scaled(u32x2_t{w[2], w[3]});
 #pragma unroll
@@ -1325,7 +1339,7 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void prefill_dma_kernel(
       asm volatile("" ::: "memory");
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
-      widen(0, 0);
+      widen(kt0, 0, 0);
       int t = 0;
       for (int kt = kt0; kt <= kt_last; kt += kKT, ++t) {
         const bool has_next = kt + kKT <= kt_last;
@@ -1339,7 +1353,7 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void prefill_dma_kernel(
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         const int st_c = t % STAGES;  // stage of tile kt (free: widened last step)
-        if (has_next) widen((t + 1) % STAGES, (t + 1) & 1);
+        if (has_next) widen(kt + kKT, (t + 1) % STAGES, (t + 1) & 1);
         const lds_u8_t *kb = kv_base + (t & 1) * 2 * TILEB;
         compute_tile(kt, kb, kb + TILEB, [&]() {
           if (kt + STAGES * kKT <= kt_last) issue8(kt + STAGES * kKT, st_c);
@@ -1354,25 +1368,48 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void prefill_dma_kernel(
     for (int i = 0; i < kAhead; ++i)
       if (kt0 + i * kKT <= kt_last) issue_tile(kt0 + i * kKT, k_at(i), k_at(i) + TILEB);
     scale_q();
-    int st = 0;
-    for (int kt = kt0; kt <= kt_last; kt += kKT) {
-      if constexpr (STAGES == 3) {
-        if (kt + kKT <= kt_last)
-          __builtin_amdgcn_s_waitcnt(waitcnt_vm(2 * NJ));  // the next tile stays in flight
-        else
+    // The tiles run in up to three stretches of this one loop: it stops before
+    // a first or last tile with keys outside [kmin, kmax), whose V rows are
+    // cleared there, so that the steps carry nothing for it.  2048 tokens of 64
+    // q / 8 kv heads, d = 64, after 4096: 186 us without the clearing, 183 like
+    // this, 202 with the test and the clearing inside a step; 777 tokens after
+    // 1536, 32 q / 8 kv heads, d = 128: 52.1, 51.7 and 53.3.
+    int st = 0, kt = kt0;
+    int stop = cut_tile(kt0) ? kt0 - kKT : cut_tile(kt_last) ? kt_last - kKT : kt_last;
+    while (true) {
+      for (; kt <= stop; kt += kKT) {
+        if constexpr (STAGES == 3) {
+          if (kt + kKT <= kt_last)
+            __builtin_amdgcn_s_waitcnt(waitcnt_vm(2 * NJ));  // the next tile stays in flight
+          else
+            __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
+        } else {
           __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
-      } else {
-        __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
+        }
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        const int st_n = st == 0 ? STAGES - 1 : st - 1;  // (st + kAhead) % STAGES
+        compute_tile(kt, kv_base + st * 2 * TILEB, kv_base + st * 2 * TILEB + TILEB, [&]() {
+          if (kt + kAhead * kKT <= kt_last)
+            issue_tile(kt + kAhead * kKT, k_at(st_n), k_at(st_n) + TILEB);
+        });
+        st = st == STAGES - 1 ? 0 : st + 1;
       }
+      if (kt > kt_last) break;
+      __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
       asm volatile("" ::: "memory");
-      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_s_barrier();  // every thread's copies of this tile are in LDS
       asm volatile("" ::: "memory");
-      const int st_n = st == 0 ? STAGES - 1 : st - 1;  // (st + kAhead) % STAGES
-      compute_tile(kt, kv_base + st * 2 * TILEB, kv_base + st * 2 * TILEB + TILEB, [&]() {
-        if (kt + kAhead * kKT <= kt_last)
-          issue_tile(kt + kAhead * kKT, k_at(st_n), k_at(st_n) + TILEB);
-      });
-      st = st == STAGES - 1 ? 0 : st + 1;
+      typedef __attribute__((address_space(3))) u32x4_t lds_u32x4_t;
+      lds_u8_t *const vb = kv_base + st * 2 * TILEB + TILEB;
+      for (int i = tid; i < kKT * CH; i += WAVES * 64) {
+        const int key = kt + i / CH;  // the swizzle stays inside a row
+        if (key < kmin || key >= kmax) *(lds_u32x4_t *)(vb + (i << 4)) = u32x4_t{0u, 0u, 0u, 0u};
+      }
+      // visible to all after the barrier of the tile's step
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      stop = kt < kt_last && cut_tile(kt_last) ? kt_last - kKT : kt_last;
     }
   }
 
