@@ -61,6 +61,53 @@ def test_plain_calls_go_direct():
         assert ops._plain(x, torch.zeros(4))
 
 
+def _project(x, w):
+    """The decode block's choice between the few-row kernel and the library."""
+    return ops.skinny_linear(x, w) if ops.skinny_linear_ok(x, w) else x @ w
+
+
+def test_few_row_projection_keeps_the_library_products_transforms(monkeypatch):
+    """Tangents, batching, gradients, subclasses and autocast are those of
+    ``x @ w``; ordinary calls take the kernel (stubbed here by the product)."""
+    calls = []
+
+    def launch(x, w, *a):
+        calls.append(type(w))
+        return torch.mm(x.detach(), w.detach())
+
+    monkeypatch.setattr(ops.K, "skinny_linear", launch)
+    g = torch.Generator().manual_seed(0)
+    x, w, t = (torch.randn(s, generator=g).to(torch.bfloat16) for s in ((4, 64), (64, 32), (64, 32)))
+
+    assert torch.equal(_project(x, w), x @ w) and len(calls) == 1
+    out, tangent = torch.func.jvp(lambda a: _project(x, a), (w,), (t,))
+    assert torch.equal(out, x @ w) and torch.equal(tangent, x @ t)
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(w, t)
+        assert torch.equal(torch.autograd.forward_ad.unpack_dual(_project(x, dual)).tangent, x @ t)
+    ws = torch.stack((w, t))
+    assert torch.equal(torch.func.vmap(lambda a: _project(x, a))(ws), torch.matmul(x, ws))
+    assert _project(x, w.clone().requires_grad_()).requires_grad
+
+    class Sub(torch.Tensor):
+        seen = []
+
+        @classmethod
+        def __torch_function__(cls, func, types, args=(), kwargs=None):
+            cls.seen.append(func.__name__)
+            return super().__torch_function__(func, types, args, kwargs or {})
+
+    _project(x, w.as_subclass(Sub))
+    assert any("matmul" in n for n in Sub.seen)
+    assert len(calls) == 1  # none of these took the kernel
+    with torch.autocast("cpu", dtype=torch.float16):
+        assert not ops.skinny_linear_ok(x, w)
+    with torch.autocast("cpu", dtype=torch.bfloat16):
+        assert ops.skinny_linear_ok(x, w)
+    compiled = torch.compile(lambda a: ops.skinny_linear_ok(x, a), backend="eager", fullgraph=True)
+    assert compiled(w)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("inference", [False, True])
 def test_direct_calls_equal_the_ops(gpu, monkeypatch, inference):

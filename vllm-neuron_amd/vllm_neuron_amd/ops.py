@@ -36,12 +36,16 @@ import torch
 from torch import Tensor
 from torch.library import custom_op
 
+from torch._subclasses.fake_tensor import FakeTensor
+from torch._subclasses.functional_tensor import FunctionalTensor
 from torch.autograd import forward_ad, graph
 
 from . import _kernels as K
 from . import _native as N
 
 _TENSOR_TYPES = (Tensor, torch.nn.Parameter)
+# what stands for such a tensor while a graph is traced
+_PRODUCT_TYPES = _TENSOR_TYPES + (FakeTensor, FunctionalTensor)
 
 
 def _plain(*tensors: Optional[Tensor]) -> bool:
@@ -525,10 +529,20 @@ def _(x, w, norm, gamma, eps, dim_actual):
 
 
 def skinny_linear_ok(x: Tensor, w: Tensor) -> bool:
-    """Shapes and strides the kernel takes, and no gradient wanted (it has
-    none; the library product does)."""
-    return K.skinny_linear_ok(x, w) and not (
-        torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))
+    """Shapes and strides the kernel takes, and nothing wanted that only the
+    library product has: a gradient or a forward-mode tangent, a batching rule
+    or another transform, a tensor subclass's own product, autocast to a
+    type other than bf16."""
+    if not K.skinny_linear_ok(x, w) or (torch.is_grad_enabled()
+                                        and (x.requires_grad or w.requires_grad)):
+        return False
+    dev = x.device.type
+    if torch.is_autocast_enabled(dev) and torch.get_autocast_dtype(dev) != torch.bfloat16:
+        return False
+    if torch.compiler.is_compiling():  # traced: x and w are plain tensors there
+        return True
+    return (forward_ad._current_level < 0 and not torch._C._are_functorch_transforms_active()
+            and type(x) in _PRODUCT_TYPES and type(w) in _PRODUCT_TYPES)
 
 
 def skinny_linear(x, w, norm: bool = False, gamma=None, eps: float = 0.0,
