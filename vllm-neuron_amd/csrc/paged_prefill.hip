@@ -1245,7 +1245,7 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void prefill_dma_kernel(
   // null block's) may hold NaN or Inf.  Their scores are masked, but 0 * V is
   // NaN there, so their V rows are cleared in LDS: by the threads that widen
   // them (FP8), or, on the first and last tile alone, between the copy and the
-  // step of the tile (one more barrier).
+  // step of the tile.
   const int kmin = readfirstlane(kr.kmin), kmax = readfirstlane(kr.kmax);
   auto cut_tile = [&](int kt) { return kt < kmin || kt + kKT > kmax; };
 
@@ -1397,15 +1397,16 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void prefill_dma_kernel(
         st = st == STAGES - 1 ? 0 : st + 1;
       }
       if (kt > kt_last) break;
+      // each lane clears what it copied itself, so its own wait is enough
       __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
-      asm volatile("" ::: "memory");
-      __builtin_amdgcn_s_barrier();  // every thread's copies of this tile are in LDS
       asm volatile("" ::: "memory");
       typedef __attribute__((address_space(3))) u32x4_t lds_u32x4_t;
       lds_u8_t *const vb = kv_base + st * 2 * TILEB + TILEB;
-      for (int i = tid; i < kKT * CH; i += WAVES * 64) {
-        const int key = kt + i / CH;  // the swizzle stays inside a row
-        if (key < kmin || key >= kmax) *(lds_u32x4_t *)(vb + (i << 4)) = u32x4_t{0u, 0u, 0u, 0u};
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        const int q = kDmaWaves * j + wave, key = kt + RPI * q + dma_r;
+        if (key < kmin || key >= kmax)
+          *(lds_u32x4_t *)(vb + q * 1024 + lane * 16) = u32x4_t{0u, 0u, 0u, 0u};
       }
       // visible to all after the barrier of the tile's step
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
