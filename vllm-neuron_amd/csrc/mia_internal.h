@@ -71,6 +71,7 @@ struct PrefillPlan {
   bool even;         // one sequence, cut evenly on the device (fp32 partials)
   int whole;         // even: row tiles left uncut
   int row_tiles;     // even: row tiles of the launch
+  int part_rows;     // even: rows of a head that have partials
   int slots;         // workgroups resident on the device at once
   size_t ws_bytes;   // workspace bytes (0 without split)
 };

@@ -56,6 +56,9 @@ constexpr int kMaxChunks = 8; // chunks of ksplit keys of a split row tile at mo
 constexpr int kMaxEven = 32;
 constexpr int kMinEvenTiles = 4;
 constexpr int part32_bytes(int D) { return 4 * D + 16; }
+// Partials of an even split at most (an unbounded plan of 1100 tokens under a
+// 262144-token table, 32 q / 8 kv heads, took 12 chunks and 223 MB).
+constexpr int64_t kMaxEvenBytes = 160 << 20;
 
 struct PrefillKParams {
   const uint16_t *q;
@@ -90,6 +93,7 @@ struct PrefillKParams {
                   // nsplit equal chunks, partials in fp32
   int whole;      // even: row tiles (of the grid's last rows) left uncut
   int row_tiles;  // even: row tiles of the grid
+  int part_rows;  // even: rows of a head that have partials (those of the cut row tiles)
   int slots;      // workgroups resident on the device at once
   int rows_wg;    // query rows per workgroup of the attention kernel
   int rows_max;   // max_seqlen_q * G
@@ -444,7 +448,7 @@ template <int D>
 MIA_DEV void store_part32(const PrefillKParams &p, const f32x16_t (&acc_o)[D / 32], float m_run,
                           float l_run, int h, int r, int half, int sp, float vscale) {
   float *w = reinterpret_cast<float *>(
-      p.ws + (((int64_t)h * p.rows_max + r) * p.nsplit + sp) * (int64_t)part32_bytes(D));
+      p.ws + (((int64_t)h * p.part_rows + r) * p.nsplit + sp) * (int64_t)part32_bytes(D));
 #pragma unroll
   for (int db = 0; db < D / 32; ++db)
 #pragma unroll
@@ -1442,7 +1446,7 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void prefill_dma_kernel(
     constexpr int DBP = D / 64;
     float *const part = reinterpret_cast<float *>(p.ws);
     const int64_t step = (int64_t)p.nsplit * (part32_bytes(D) / 4);
-    const int64_t first = ((int64_t)h * p.rows_max + row0 + wave * kRowsW) * step +
+    const int64_t first = ((int64_t)h * p.part_rows + row0 + wave * kRowsW) * step +
                           (int64_t)sp * (part32_bytes(D) / 4);
 #pragma unroll
     for (int pass = 0; pass < 2; ++pass) {
@@ -1623,7 +1627,7 @@ __global__ __launch_bounds__(256) void prefill_merge32_kernel(PrefillKParams p) 
   const int pos_r = r / p.G;
   const int hq = h * p.G + (r - pos_r * p.G);
   const int c8 = (lane % LPR) * 8;
-  const uint8_t *w0 = p.ws + ((int64_t)h * p.rows_max + r) * p.nsplit * (int64_t)PB;
+  const uint8_t *w0 = p.ws + ((int64_t)h * p.part_rows + r) * p.nsplit * (int64_t)PB;
   const float sink2 = p.sink ? p.sink[hq] * kLog2e : -INFINITY;
   float M = sink2, L = p.sink ? 1.0f : 0.f;  // the sink joins the denominator
   float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -1760,6 +1764,9 @@ void plan_even(const mia_prefill_args &a, bool half_ok, PrefillPlan &pl) {
   };
   double best = pl.nsplit > 1 ? cut8(R, pl.nsplit, T, part_bytes(D)) : 1e30;
   auto offer = [&](double est, int n, int whole, int waves, int rows) {
+    const int64_t tiles = (pl.rows_max + rows - 1) / rows;
+    const int64_t cut = std::min<int64_t>(pl.rows_max, (tiles - whole) * rows);
+    if (n > 1 && Hkv * cut * n * part32_bytes(D) > kMaxEvenBytes) return;
     if (est >= (n > 1 || !pl.even ? 0.95 : 1.0) * best) return;
     pl.even = true;
     best = est;
@@ -1791,7 +1798,8 @@ void plan_even(const mia_prefill_args &a, bool half_ok, PrefillPlan &pl) {
   if (!pl.even) return;
   pl.ksplit = 1 << 30;
   pl.row_tiles = (pl.rows_max + pl.rows_wg - 1) / pl.rows_wg;
-  pl.ws_bytes = pl.nsplit > 1 ? (size_t)Hkv * pl.rows_max * pl.nsplit * part32_bytes(D) : 0;
+  pl.part_rows = std::min(pl.rows_max, (pl.row_tiles - pl.whole) * pl.rows_wg);
+  pl.ws_bytes = pl.nsplit > 1 ? (size_t)Hkv * pl.part_rows * pl.nsplit * part32_bytes(D) : 0;
 }
 
 }  // namespace
@@ -1902,6 +1910,7 @@ int launch_paged_prefill(const mia_prefill_args &a, const PrefillPlan &pl, hipSt
   kp.even = pl.even ? 1 : 0;
   kp.whole = pl.whole;
   kp.row_tiles = pl.row_tiles;
+  kp.part_rows = pl.part_rows;
   kp.slots = pl.slots;
   kp.num_seqs = a.num_seqs;
   kp.rows_wg = pl.rows_wg;
@@ -1981,7 +1990,7 @@ int launch_paged_prefill(const mia_prefill_args &a, const PrefillPlan &pl, hipSt
   if (rc || pl.nsplit <= 1) return rc;
   if (pl.even) {
     const int rows = 4 * 64 / (a.head_dim / 8);  // per workgroup
-    const dim3 mgrid((unsigned)((pl.rows_max + rows - 1) / rows), (unsigned)a.num_kv_heads, 1u);
+    const dim3 mgrid((unsigned)((pl.part_rows + rows - 1) / rows), (unsigned)a.num_kv_heads, 1u);
     if (a.head_dim == 128)
       hipLaunchKernelGGL((prefill_merge32_kernel<128>), mgrid, dim3(256), 0, s, kp);
     else
