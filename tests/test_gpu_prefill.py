@@ -9,6 +9,8 @@ from vllm_neuron_amd import _kernels as K
 from vllm_neuron_amd import workloads as W
 from vllm_neuron_amd.functional import mixed_batch_attention, segmented_attention
 
+from test_prefill_plan import even_bytes, workspace_bytes
+
 pytestmark = pytest.mark.gpu
 
 TOL_BF16 = 2e-2
@@ -400,15 +402,18 @@ def test_copy_ring_tile_edges_and_rising_scores(gpu, d, bs, new, prior, window, 
 
 
 EVEN_CASES = [
-    # q heads, kv heads, d, bs, new, prior, table tokens, window, sink, fp8
-    (8, 2, 128, 32, 1, 4096, 0, 0, False, False),      # one row, 4-wave workgroups
-    (32, 8, 128, 16, 200, 5000 // 16 * 16, 0, 0, True, False),   # 8-wave, 8 chunks
-    (32, 8, 128, 32, 65, 640, 16384, 0, True, False),  # table far wider than the sequence
-    (8, 1, 64, 64, 33, 9600, 0, 0, True, False),       # 32 chunks, one kv head
-    (64, 8, 64, 32, 1100, 4096, 0, 0, True, False),    # whole rounds of uncut row tiles
-    (32, 8, 64, 16, 130, 6000 // 16 * 16, 0, 1500, False, False),  # window cut across chunks
-    (12, 2, 128, 64, 100, 4096, 0, 0, False, True),    # FP8 ring
-    (12, 2, 64, 64, 100, 4096, 0, 0, True, True),      # FP8, register-staged kernel
+    # q heads, kv heads, d, bs, new, prior, table tokens, window, sink, fp8, rows cut, chunks
+    (8, 2, 128, 32, 1, 4096, 0, 0, False, False, 4, 16),      # one row, 4-wave workgroups
+    (32, 8, 128, 16, 200, 5000 // 16 * 16, 0, 0, True, False, 800, 6),   # 4-wave, 6 chunks
+    (32, 8, 128, 32, 500, 8800, 0, 0, True, False, 2000, 4),  # 8-wave, 4 chunks
+    (32, 8, 128, 32, 65, 640, 16384, 0, True, False, 260, 12),  # table far wider than the sequence
+    (64, 8, 64, 32, 400, 288, 131072, 0, True, False, 3200, 12),  # the same, 8-wave, d = 64
+    (8, 1, 64, 64, 33, 9600, 0, 0, True, False, 264, 32),     # 32 chunks, one kv head
+    (64, 8, 64, 32, 1100, 4096, 0, 0, True, False, 768, 6),   # whole rounds of uncut row tiles
+    (32, 8, 64, 16, 130, 6000 // 16 * 16, 0, 1500, False, False, 520, 4),  # window cut across chunks
+    (12, 2, 128, 64, 100, 4096, 0, 0, False, True, 600, 16),  # FP8 ring
+    (12, 2, 64, 64, 100, 4096, 0, 0, True, True, 600, 16),    # FP8, register-staged kernel
+    (48, 8, 128, 64, 1536, 1088, 16384, 0, False, True, 1024, 6),  # FP8, 4 of 36 row tiles cut
 ]
 
 
@@ -417,7 +422,7 @@ def test_single_sequence_even_split(gpu, case):
     """One sequence whose row tiles are cut evenly on the device: equal to the
     uncut launch within two bf16 steps (each chunk keeps its own running
     maximum; partials are fp32), and within tolerance of float64 math."""
-    Hq, Hkv, d, bs, new, prior, wide, win, use_sink, fp8 = EVEN_CASES[case]
+    Hq, Hkv, d, bs, new, prior, wide, win, use_sink, fp8, rows, chunks = EVEN_CASES[case]
     cfg = W.PrefillConfig("e", 1, Hq, Hkv, d, bs, new, prior, prior, fp8=fp8, seed=170 + case)
     b = W.make_prefill_batch(cfg, gpu)
     kw = {}
@@ -431,6 +436,8 @@ def test_single_sequence_even_split(gpu, case):
     if wide:
         table = torch.full((1, wide // bs), -1, dtype=torch.int32, device=gpu)
         table[:, :b.block_table.shape[1]] = b.block_table
+    keys = table.shape[1] * bs
+    assert workspace_bytes(Hq, Hkv, d, bs, new, keys, fp8, win) == even_bytes(Hkv, d, rows, chunks)
     sink = torch.randn(Hq, generator=torch.Generator().manual_seed(case)).to(gpu) if use_sink else None
     run = lambda split: K.paged_prefill(b.q, b.cu_seqlens, b.prior, new, b.k_cache, b.v_cache, table,
                                         scale=d ** -0.5, sliding_window=win, sink=sink,

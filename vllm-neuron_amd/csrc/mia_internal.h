@@ -72,6 +72,7 @@ struct PrefillPlan {
   int whole;         // even: row tiles left uncut
   int row_tiles;     // even: row tiles of the launch
   int part_rows;     // even: rows of a head that have partials
+  uint64_t n_len;    // even: chunks for shorter sequences, 5 bits per length class
   int slots;         // workgroups resident on the device at once
   size_t ws_bytes;   // workspace bytes (0 without split)
 };

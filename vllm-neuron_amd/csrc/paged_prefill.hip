@@ -55,6 +55,9 @@ constexpr int kMaxChunks = 8; // chunks of ksplit keys of a split row tile at mo
 // padding.
 constexpr int kMaxEven = 32;
 constexpr int kMinEvenTiles = 4;
+constexpr int kEvenClass0 = 3;    // bits of kMinEvenTiles
+constexpr int kEvenClasses = 12;  // 5 bits each in a 64-bit word
+static_assert(kMinEvenTiles == 1 << (kEvenClass0 - 1) && kMaxEven <= 32, "even_chunks");
 constexpr int part32_bytes(int D) { return 4 * D + 16; }
 // Partials of an even split at most (an unbounded plan of 1100 tokens under a
 // 262144-token table, 32 q / 8 kv heads, took 12 chunks and 223 MB).
@@ -94,6 +97,7 @@ struct PrefillKParams {
   int whole;      // even: row tiles (of the grid's last rows) left uncut
   int row_tiles;  // even: row tiles of the grid
   int part_rows;  // even: rows of a head that have partials (those of the cut row tiles)
+  uint64_t n_len; // even: chunks by the sequence's length (even_chunks)
   int slots;      // workgroups resident on the device at once
   int rows_wg;    // query rows per workgroup of the attention kernel
   int rows_max;   // max_seqlen_q * G
@@ -155,6 +159,15 @@ MIA_DEV bool row_range(const PrefillKParams &p, int prior, int kvl, int pos, int
   return uni;
 }
 
+// Even split: chunks of a cut row tile (before its own length limits them) of
+// a sequence of kvl keys.  The host plans for the table's width; a shorter
+// sequence takes the count that the host chose for its length: 5 bits (count -
+// 1) per power of two of key tiles, from kMinEvenTiles .. 2 kMinEvenTiles - 1 on.
+MIA_DEV int even_chunks(const PrefillKParams &p, int kvl) {
+  const int cls = 32 - __builtin_clz(max((kvl + kKT - 1) / kKT, 1)) - kEvenClass0;
+  return (int)(p.n_len >> (5 * min(max(cls, 0), kEvenClasses - 1)) & 31u) + 1;
+}
+
 // Key range of the workgroup whose rows start at row0 (rows are GQA-packed:
 // row = pos * G + g): the keys some row sees, the keys every row sees, the
 // tiles and the number of key chunks.  Shared by the attention and merge
@@ -195,11 +208,12 @@ MIA_DEV KeyRange wg_key_range(const PrefillKParams &p, int seq, int prior, int S
   k.any = k.kmax > k.kmin;
   k.kt0 = (k.kmin / kKT) * kKT;
   k.kt_last = k.kmax > k.kt0 ? ((k.kmax - 1) / kKT) * kKT : k.kt0;
-  if (p.even)
+  if (p.even) {
+    const int n = even_chunks(p, kvl);
     k.n_sp = k.any && row0 / p.rows_wg < p.row_tiles - p.whole
-                 ? min(max(((k.kt_last - k.kt0) / kKT + 1) / kMinEvenTiles, 1), p.nsplit)
+                 ? min(max(((k.kt_last - k.kt0) / kKT + 1) / kMinEvenTiles, 1), n)
                  : 1;
-  else
+  } else
     k.n_sp = (k.any && p.nsplit > 1) ? k.kt_last / ksplit - k.kt0 / ksplit + 1 : 1;
   return k;
 }
@@ -229,9 +243,13 @@ MIA_DEV void chunk_tiles(const PrefillKParams &p, const KeyRange &k, int ksplit,
 // within each XCD.  When the group count is not a multiple of 8 the launch
 // order is kept.
 // One sequence with an even split: a group's items are its uncut row tiles,
-// then the chunks of the others, tile by tile (grid.x = whole + (row tiles -
-// whole) * nsplit).
-MIA_DEV uint3 xcd_tile(const PrefillKParams &p) {
+// then the n chunks of the others, tile by tile (grid.x = whole + (row tiles -
+// whole) * nsplit; n <= nsplit, what is left over exits).  Every n-th workgroup
+// of nsplit places per tile instead would sit on a few CUs of the dispatcher's
+// round over the shader engines (1500 tokens after 4000, table of 65536 keys:
+// 389 us for 152); chunk by chunk starts heavy chunks late (2048 tokens, 8 q /
+// 2 kv heads: 38.3 us for 34.7).
+MIA_DEV uint3 xcd_tile(const PrefillKParams &p, int n_even) {
   constexpr uint32_t X = 8;
   const uint32_t R = gridDim.x;                 // row tiles per group
   const uint32_t groups = gridDim.y * gridDim.z;
@@ -243,11 +261,12 @@ MIA_DEV uint3 xcd_tile(const PrefillKParams &p) {
     g = (k / R) * X + x;
   }
   if (p.even) {
-    const uint32_t W = (uint32_t)p.whole, n = (uint32_t)p.nsplit;
+    const uint32_t W = (uint32_t)p.whole, n = (uint32_t)n_even;
+    const uint32_t j = rt < W ? rt : W + (rt - W) / n;
     uint3 t;
-    t.x = (uint32_t)p.row_tiles - 1 - (rt < W ? rt : W + (rt - W) / n);
+    t.x = (uint32_t)p.row_tiles - 1 - min(j, (uint32_t)p.row_tiles - 1);
     t.y = g % gridDim.y;
-    t.z = rt < W ? 0 : (rt - W) % n;
+    t.z = rt < W ? 0 : j < (uint32_t)p.row_tiles ? (rt - W) % n : kMaxEven;  // past every n_sp
     return t;
   }
   // heaviest row tile first: under the causal mask the last rows see the
@@ -353,9 +372,13 @@ MIA_DEV uint3 ranked_tile(const PrefillKParams &p, int *scratch, int cap, SeqInf
   const uint32_t n_x = R * (groups / X);  // items per XCD
   // LDS: costs [0, n_x), the chosen item at [n_x], item metadata from mo
   const uint32_t mo = (n_x + 4) & ~3u;
+  if (p.even) {
+    info = load_seq(p, 0);
+    return xcd_tile(p, even_chunks(p, seq_kv_len(p, 0, info.prior, info.S_q)));
+  }
   if (!p.rank_items || groups % X != 0 || mo + 4 * n_x > (uint32_t)cap || n_x > kRankMax ||
       n_x > NT) {
-    const uint3 t = xcd_tile(p);
+    const uint3 t = xcd_tile(p, 1);
     info = load_seq(p, (int)(t.z % (uint32_t)p.num_seqs));
     return t;
   }
@@ -1717,10 +1740,9 @@ bool use_dma_kernel(const mia_prefill_args &a) {
 namespace {
 
 // Launch of one sequence.  The host knows the new tokens and, from the table's
-// width, the most keys a row tile can see; a row tile that sees fewer is cut
-// into fewer chunks by the kernel (kMinEvenTiles).  Uncut, a short chunk after a
-// long context is a few workgroups that each walk the whole context: 200 tokens
-// after 8000 (32 q / 8 kv heads, d = 128) took 208 us on 32 of 256 CUs.
+// width, the most keys a row tile can see.  Uncut, a short chunk after a long
+// context is a few workgroups that each walk the whole context: 200 tokens
+// after 8000 (32 q / 8 kv heads, d = 128) took 204 us on 32 of 256 CUs.
 //
 // Choices: 8-wave workgroups (256 rows, one per CU) with every row tile cut
 // into n chunks, or only the row tiles left over after whole rounds of uncut
@@ -1731,10 +1753,13 @@ namespace {
 // workgroup (FP8 1.85), 1.27 us for a 4-wave one alone on its CU and 2.1 us for
 // two; d = 64, 1.0 / 0.75 / 1.15 us.  Start and epilogue of an item take ~6 us.
 // A plan of ksplit-key chunks already in pl (a long table under few row tiles)
-// keeps its bf16 partials and is taken unless another choice is 5 % better.
-// Measured before and now (us; new tokens after prior ones): 777 / 1536 64 -> 52,
-// 200 / 8000 125 -> 49, 64 / 16000 213 -> 41 (llama-like, d = 128, 32 q / 8 kv);
-// 100 / 4096 51 -> 22, 1200 / 12000 409 -> 299 (d = 64); FP8 300 / 4096 89 -> 58.
+// keeps its bf16 partials unless another choice is 5 % better, and so does
+// every choice against one with more chunks.
+//
+// A table may be far wider than its sequence: the launch shape is planned for
+// the width, the chunk count again for every power of two of the real length
+// (even_chunks).  With the width's count a sequence of 1600 keys (1100 new, 32 q
+// / 8 kv heads, d = 128) under a 131072-key table took 80 us, 52 without a split.
 void plan_even(const mia_prefill_args &a, bool half_ok, PrefillPlan &pl) {
   const int D = a.head_dim;
   const double t8 = a.cache_dtype != MIA_DTYPE_BF16 ? 1.85 : D == 128 ? 1.6 : 1.0;
@@ -1747,22 +1772,40 @@ void plan_even(const mia_prefill_args &a, bool half_ok, PrefillPlan &pl) {
   double keys = (double)a.blocks_per_seq * a.block_size;
   if (!a.non_causal && a.sliding_window > 0)
     keys = std::min(keys, a.sliding_window + (double)rows8 * Hkv / a.num_q_heads + kKT - 1);
-  const double drop =
-      a.non_causal || a.sliding_window > 0 ? 0.0 : std::min<double>(a.max_seqlen_q, keys) / kKT;
   const double T = std::max(1.0, keys / kKT);
+  auto drop_of = [&](double T) {
+    return a.non_causal || a.sliding_window > 0 ? 0.0
+                                                : std::min((double)a.max_seqlen_q / kKT, T);
+  };
   const int R = (pl.rows_max + rows8 - 1) / rows8, R4 = (pl.rows_max + 127) / 128;
+  const int per_head = std::max(1, cus / Hkv);  // row tiles of a head in one round
   auto merge = [&](double rows, int n, int row_bytes) {
     return n > 1 ? 6.0 + std::min<double>(rows, pl.rows_max) * Hkv * n * row_bytes * 2 / 4.5e6
                  : 0.0;
   };
-  // 8-wave workgroups: the last `cut` row tiles in n chunks
-  auto cut8 = [&](int cut, int n, double far, int row_bytes) {
+  // 8-wave workgroups: the last `cut` row tiles in n chunks, the longest of `far` tiles
+  auto cut8 = [&](int cut, int n, double far, double drop, int row_bytes) {
     const double mean = std::max(1.0, far - drop * cut / R / 2);
     const double rounds = std::ceil((double)cut * n * Hkv / cus);
     return std::max(far / n, rounds * mean / n) * t8 + rounds * fixed +
            merge((double)cut * rows8, n, row_bytes);
   };
-  double best = pl.nsplit > 1 ? cut8(R, pl.nsplit, T, part_bytes(D)) : 1e30;
+  auto est8 = [&](int n, int whole, double T) {
+    const double drop = drop_of(T);
+    return (whole ? whole / per_head * (T * t8 + fixed) : 0.0) +
+           cut8(R - whole, n, T - drop * whole / R, drop, part32_bytes(D));
+  };
+  auto est4 = [&](int n, double T) {
+    // whole rounds of two per CU, heavy items beside light ones, then the rest
+    const double mean = std::max(1.0, T - drop_of(T) / 2), len = (T + mean) / 2 / n;
+    const double fill = (double)R4 * n * Hkv / cus;  // workgroups per CU
+    const double full = std::floor(fill / 2), rest = fill - 2 * full;
+    const double t = rest > 0 ? t4 + (t4x2 - t4) * std::max(0.0, rest - 1) : 0.0;
+    return std::max(T / n * t4, len * (full * t4x2 + t)) + std::ceil(fill / 2) * fixed +
+           merge((double)pl.rows_max, n, part32_bytes(D));
+  };
+  auto next = [](int n) { return n + (n < 4 ? 1 : n < 8 ? 2 : n < 16 ? 4 : 8); };
+  double best = pl.nsplit > 1 ? cut8(R, pl.nsplit, T, drop_of(T), part_bytes(D)) : 1e30;
   auto offer = [&](double est, int n, int whole, int waves, int rows) {
     const int64_t tiles = (pl.rows_max + rows - 1) / rows;
     const int64_t cut = std::min<int64_t>(pl.rows_max, (tiles - whole) * rows);
@@ -1775,31 +1818,38 @@ void plan_even(const mia_prefill_args &a, bool half_ok, PrefillPlan &pl) {
     pl.dma_waves = waves;
     pl.rows_wg = rows;
   };
-  const int per_head = std::max(1, cus / Hkv);  // row tiles of a head in one round
-  for (int n = 1; n <= kMaxEven; n += n < 4 ? 1 : n < 8 ? 2 : n < 16 ? 4 : 8) {
+  for (int n = 1; n <= kMaxEven; n = next(n)) {
     if (n > 1 && T / n < kMinEvenTiles) break;
-    for (const int whole : {0, (R - 1) / per_head * per_head}) {
-      if (whole && n == 1) continue;
-      offer((whole ? whole / per_head * (T * t8 + fixed) : 0.0) +
-                cut8(R - whole, n, T - drop * whole / R, part32_bytes(D)),
-            n, whole, kDmaWaves, rows8);
-    }
-    if (half_ok) {
-      // whole rounds of two per CU, heavy items beside light ones, then the rest
-      const double mean = std::max(1.0, T - drop / 2), len = (T + mean) / 2 / n;
-      const double fill = (double)R4 * n * Hkv / cus;  // workgroups per CU
-      const double full = std::floor(fill / 2), rest = fill - 2 * full;
-      const double t = rest > 0 ? t4 + (t4x2 - t4) * std::max(0.0, rest - 1) : 0.0;
-      offer(std::max(T / n * t4, len * (full * t4x2 + t)) + std::ceil(fill / 2) * fixed +
-                merge((double)pl.rows_max, n, part32_bytes(D)),
-            n, 0, 4, 128);
-    }
+    for (const int whole : {0, (R - 1) / per_head * per_head})
+      if (!whole || n > 1) offer(est8(n, whole, T), n, whole, kDmaWaves, rows8);
+    if (half_ok) offer(est4(n, T), n, 0, 4, 128);
   }
   if (!pl.even) return;
   pl.ksplit = 1 << 30;
   pl.row_tiles = (pl.rows_max + pl.rows_wg - 1) / pl.rows_wg;
   pl.part_rows = std::min(pl.rows_max, (pl.row_tiles - pl.whole) * pl.rows_wg);
   pl.ws_bytes = pl.nsplit > 1 ? (size_t)Hkv * pl.part_rows * pl.nsplit * part32_bytes(D) : 0;
+  pl.n_len = 0;
+  // chunks that fill the device once are taken in any case (400 tokens after
+  // 1536, 32 q / 8 kv heads, table of 8192 keys: 37 us, 40 with the estimate's)
+  const int fill = cus / std::max(1, (pl.row_tiles - pl.whole) * Hkv);
+  for (int c = 0; c < kEvenClasses; ++c) {
+    // lengths of 2^(c + 2) .. 2^(c + 3) - 1 tiles: the count for their middle
+    const double L = 0.75 * (1 << (c + kEvenClass0));
+    int n_best = 1;
+    double t_best = 1e30;
+    for (int n = 1; n <= pl.nsplit; n = next(n)) {
+      if (n > 1 && L / n < kMinEvenTiles) break;
+      const double est = pl.dma_waves == 4 && half_ok ? est4(n, L) : est8(n, pl.whole, L);
+      if (est >= (n > 1 ? 0.95 : 1.0) * t_best) continue;
+      t_best = est;
+      n_best = n;
+    }
+    const int most = ((1 << (c + kEvenClass0)) - 1) / kMinEvenTiles;
+    n_best = std::max(n_best, std::min({pl.nsplit, fill, most}));
+    if (L * 4 / 3 > T || (a.sliding_window > 0 && !a.non_causal)) n_best = pl.nsplit;
+    pl.n_len |= (uint64_t)(n_best - 1) << (5 * c);
+  }
 }
 
 }  // namespace
@@ -1911,6 +1961,7 @@ int launch_paged_prefill(const mia_prefill_args &a, const PrefillPlan &pl, hipSt
   kp.whole = pl.whole;
   kp.row_tiles = pl.row_tiles;
   kp.part_rows = pl.part_rows;
+  kp.n_len = pl.n_len;
   kp.slots = pl.slots;
   kp.num_seqs = a.num_seqs;
   kp.rows_wg = pl.rows_wg;
