@@ -340,10 +340,11 @@ typedef struct {
   void *workspace;
   size_t workspace_bytes;
   int32_t split_tokens;
-  /* Below head_dim and a multiple of 8: the q and out rows hold only this many
-   * channels (none past it is read or written) and the cache rows are zero
-   * from there on, i.e. the caller padded a narrower K and V to head_dim.
-   * Any other value (0): every row holds head_dim channels. */
+  /* Below head_dim (and a multiple of 8): the q and out rows hold only this
+   * many channels (none past it is read or written) and the cache rows are
+   * zero from there on, i.e. the caller padded a narrower K and V to head_dim.
+   * 0, or head_dim and more: every row holds head_dim channels.  Negative, or
+   * narrower and no multiple of 8: MIA_ERR_VALUE. */
   int32_t head_dim_used;
   /* Generalised visibility for dense attention (attention_cte.py:47-186,
    * flash_attention :189-343); all zero / NULL keeps the rule above.

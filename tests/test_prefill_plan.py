@@ -12,7 +12,8 @@ def even_bytes(Hkv, d, cut_rows, chunks):
     return Hkv * cut_rows * chunks * (4 * d + 16)
 
 
-def workspace_bytes(Hq, Hkv, d, bs, new, table, fp8=False, window=0, **over):
+def prefill_args(Hq, Hkv, d, bs, new, table, fp8=False, window=0):
+    """Arguments of one sequence over contiguous tensors (addresses made up)."""
     a = N.PrefillArgs()
     a.q = a.cu_seqlens_q = a.prior_tokens = a.k_cache = a.v_cache = a.block_table = a.out = 1 << 20
     a.q_stride = a.out_stride = (Hq * d, d, 1)
@@ -25,9 +26,11 @@ def workspace_bytes(Hq, Hkv, d, bs, new, table, fp8=False, window=0, **over):
     a.bt_stride = (table // bs, 0, 1)
     a.num_q_heads, a.num_kv_heads, a.head_dim, a.scale = Hq, Hkv, d, 0.1
     a.sliding_window = window
-    for k, v in over.items():
-        setattr(a, k, v)
-    n = N.lib().mia_prefill_workspace_bytes(ctypes.byref(a))
+    return a
+
+
+def workspace_bytes(*shape, **kw):
+    n = N.lib().mia_prefill_workspace_bytes(ctypes.byref(prefill_args(*shape, **kw)))
     err = N.lib().mia_last_error()
     assert not err, err.decode()
     return n
@@ -56,3 +59,16 @@ def test_even_split_workspace_is_bounded(new, table, Hq, Hkv, d, fp8):
     bf16 halves (2 d + 16 bytes a row)."""
     halves = 2 * Hkv * new * (Hq // Hkv) * (2 * d + 16)
     assert workspace_bytes(Hq, Hkv, d, 128, new, table, fp8) <= max(160 << 20, halves)
+
+
+@pytest.mark.parametrize("used, ok", [(0, True), (8, True), (120, True), (128, True), (200, True),
+                                      (-8, False), (-1, False), (4, False), (100, False), (127, False)])
+def test_head_dim_used_is_checked(used, ok):
+    """A width that the kernels cannot honour is refused: taken as the full
+    128 channels, rows of 100 would be read and written past their end."""
+    a = prefill_args(8, 2, 128, 32, 64, 2048)
+    a.head_dim_used = used
+    a.num_tokens = 0  # nothing is launched
+    rc = N.lib().mia_paged_prefill(ctypes.byref(a), None)
+    assert (rc == 0) == ok
+    assert ok or b"head_dim_used" in N.lib().mia_last_error()

@@ -331,6 +331,9 @@ static int validate_prefill(const mia_prefill_args *a) {
               MIA_ERR_VALUE, "GQA requires q_heads divisible by kv_heads");
   MIA_REQUIRE(a->head_dim == 64 || a->head_dim == 128, MIA_ERR_NOT_IMPLEMENTED,
               "prefill: head_dim must be 64 or 128");
+  MIA_REQUIRE(a->head_dim_used >= 0 &&
+                  (a->head_dim_used >= a->head_dim || a->head_dim_used % 8 == 0),
+              MIA_ERR_VALUE, "prefill: head_dim_used must be 0, a multiple of 8 or the head_dim");
   MIA_REQUIRE(a->cache_dtype == MIA_DTYPE_BF16 ||
                   a->cache_dtype == MIA_DTYPE_FP8_E4M3FN,
               MIA_ERR_NOT_IMPLEMENTED, "prefill: cache dtype must be bf16 or fp8");

@@ -1713,10 +1713,11 @@ int device_cus() {
   return cache[dev];
 }
 
-// Channels of a q / out row (below head_dim: the caller padded the cache).
+// Channels of a q / out row (below head_dim, a multiple of 8: the caller padded
+// the cache; else 0 or at least head_dim, checked by the C entry).
 int prefill_head_dim_used(const mia_prefill_args &a) {
   const int u = a.head_dim_used;
-  return u > 0 && u < a.head_dim && u % 8 == 0 ? u : a.head_dim;
+  return u > 0 && u < a.head_dim ? u : a.head_dim;
 }
 
 bool use_dma_kernel(const mia_prefill_args &a) {
