@@ -108,6 +108,23 @@ def test_few_row_projection_keeps_the_library_products_transforms(monkeypatch):
     assert compiled(w)
 
 
+@pytest.mark.parametrize("k, n, few", [
+    (256, 32, True), (2880, 32, True), (2880, 8192, True), (2048, 8224, False), (2048, 48, False),
+    (2912, 3040, False), (2912, 3072, True), (4096, 3072, True), (4096, 2880, False),
+    (4096, 6144, True), (4096, 8192, False), (4128, 3072, False), (8192, 1024, False),
+    (8192, 4096, True), (8192, 4064, False), (16384, 32, False), (16384, 6144, True),
+    (16384, 6176, False),
+])
+def test_few_row_projection_sizes(k, n, few):
+    """The kernel where it measured faster: few rows of K, or columns enough
+    for every CU and fewer than the library streams as fast."""
+    w = torch.empty(k, n, dtype=torch.bfloat16, device="meta")
+    for T in (1, 16):
+        x = torch.empty(T, k, dtype=torch.bfloat16, device="meta")
+        assert ops.K.skinny_linear_ok(x, w) == few
+    assert not ops.K.skinny_linear_ok(torch.empty(17, k, dtype=torch.bfloat16, device="meta"), w)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("inference", [False, True])
 def test_direct_calls_equal_the_ops(gpu, monkeypatch, inference):

@@ -25,7 +25,9 @@
 // 2048 x 2048 8.8 -> 7.2, 4096 x 4096 21.9 -> 19.0.  64 columns per workgroup
 // (whole lines, half the workgroups): 2048 x 3072 with norm 11.7; nontemporal
 // weight loads 13.8.  Past N = 8192 (more than one workgroup per CU) the
-// library is faster: 8192 x 10240 53.8 against 89.9.
+// library is faster: 8192 x 10240 53.8 against 89.9.  A deep K with few columns
+// leaves CUs idle: 8192 x 1024 with norm 39.5 against 34.2 at T = 8, 16384 x 32
+// 41.9 against 29.0 at T = 16; the wrapper's rule keeps those on the library.
 #include "mia_device.h"
 #include "mia_internal.h"
 

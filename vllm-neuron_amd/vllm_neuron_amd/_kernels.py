@@ -938,13 +938,11 @@ def row_norm(x: torch.Tensor, mode: int, eps: float, gamma: Optional[torch.Tenso
     return out.reshape(shape)
 
 
-def skinny_linear_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """Does ``skinny_linear`` take ``x [T, K]`` and ``w [K, N]``, and faster
-    than a library GEMM?  At most 16 rows (one MFMA row block; from 17 rows on
-    the weights would be read twice), whole 32-column and 32-row steps, at most
-    8192 columns (one workgroup of 32 per CU: at 10240 the library is faster,
-    54 against 90 us; at 8192 x 1024 the two are equal).  Strides only:
-    addresses are not known while tracing (see ``skinny_linear``)."""
+def _skinny_takes(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Does ``skinny_linear`` take ``x [T, K]`` and ``w [K, N]``?  At most 16
+    rows (one MFMA row block; from 17 rows on the weights would be read twice),
+    whole 32-column and 32-row steps, at most 8192 columns (one workgroup of 32
+    per CU).  Strides only: addresses are not known while tracing."""
     return (x.dim() == 2 and w.dim() == 2 and x.dtype == torch.bfloat16
             and w.dtype == torch.bfloat16 and 0 < x.shape[0] <= 16 and x.shape[1] == w.shape[0]
             and x.shape[1] % 32 == 0 and w.shape[1] % 32 == 0 and 0 < w.shape[1] <= 8192
@@ -953,14 +951,30 @@ def skinny_linear_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
             and w.stride(0) >= w.shape[1] and (x.shape[0] == 1 or x.stride(0) >= x.shape[1]))
 
 
+def skinny_linear_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Does ``skinny_linear`` take the product, and faster than a library GEMM
+    after ``row_norm``?  A workgroup walks all K rows of its 32 columns, so a
+    deep K needs columns enough to keep the CUs busy, and near 8192 of them
+    the library streams as fast.  Measured at 1, 4, 8 and 16 rows on cold
+    weights (library / kernel time, without the norm; with it 0.1-0.5 better
+    at most sizes): K <= 2880 1.0-2.8 at 32 to 8192 columns (0.8 and 0.9 at
+    1024 x 512 and 512 x 1024 alone); 4096 x 3072-6144 1.08-1.24, x 512-2880
+    0.89-1.08, x 8192 0.95; 5120 to 14336 x 4096-6144 1.04-1.28, x 2048-3072
+    0.81-1.07, x 7168 0.92-1.03; 8192 x 32-1024 0.84-1.74."""
+    if not _skinny_takes(x, w):
+        return False
+    k, n = w.shape
+    return k <= 2880 or (3072 if k <= 4096 else 4096) <= n <= 6144
+
+
 def skinny_linear(x: torch.Tensor, w: torch.Tensor, norm: bool = False,
                   gamma: Optional[torch.Tensor] = None, eps: float = 0.0,
                   dim_actual: int = 0) -> torch.Tensor:
-    """``x [T, K] @ w [K, N]`` for T <= 16 (``skinny_linear_ok``), with
+    """``x [T, K] @ w [K, N]`` for T <= 16 (``_skinny_takes``), with
     ``norm`` of the RMS-normalised rows (``row_norm`` mode 1).  Rows whose
     address is not vector aligned are copied first."""
     dev = N.require_gpu(x, w)
-    if not skinny_linear_ok(x, w):
+    if not _skinny_takes(x, w):
         raise NotImplementedError("skinny_linear: unsupported shapes, strides or dtypes")
     if x.data_ptr() % 16:
         x = x.clone()
