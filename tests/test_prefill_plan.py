@@ -72,3 +72,24 @@ def test_head_dim_used_is_checked(used, ok):
     rc = N.lib().mia_paged_prefill(ctypes.byref(a), None)
     assert (rc == 0) == ok
     assert ok or b"head_dim_used" in N.lib().mia_last_error()
+
+
+@pytest.mark.parametrize("d, fp8", [(64, False), (128, False), (128, True)])
+@pytest.mark.parametrize("bs", [32, 256])
+def test_large_token_strides_keep_64_bit_offsets(d, fp8, bs):
+    """A view whose tokens lie so far apart that a block spans 2^31 bytes runs
+    the register-staged kernel (64-bit offsets) and not the copy ring: its plan
+    is that of other strides the ring does not take, below that the ring's."""
+    def plan(k_tok, v_tok, split=0):
+        a = prefill_args(32, 8, d, bs, 300, 8192, fp8)
+        a.split_tokens = split
+        a.k_cache_stride = (d, 0, k_tok, 1, 0)
+        a.v_cache_stride = (d, 0, v_tok, 1)
+        n = N.lib().mia_prefill_workspace_bytes(ctypes.byref(a))
+        assert not N.lib().mia_last_error()
+        return n
+
+    far = (1 << 31) // ((1 if fp8 else 2) * max(bs, 64))
+    near, staged = plan(far - 16, far - 16), plan(far - 16, far - 32)
+    assert near != staged  # the two kernels are told apart
+    assert plan(far, far) == staged

@@ -1730,6 +1730,10 @@ bool use_dma_kernel(const mia_prefill_args &a) {
   // d = 64: bf16 caches.  Compact launches and FP8 caches of that head dim
   // keep the register-staged kernel.
   const bool dim_ok = a.head_dim == 128 || (a.cache_dtype == MIA_DTYPE_BF16 && !a.compact_kernel);
+  // the ring holds byte offsets inside a block in 32 bits (the register-staged
+  // kernel forms them in 64): a token-major view of a large pool passes them
+  const int64_t eb = a.cache_dtype == MIA_DTYPE_BF16 ? 2 : 1;
+  if (k_tok * eb * std::max<int64_t>(a.block_size, kKT) >= ((int64_t)1 << 31)) return false;
   return dim_ok && dtype_ok && a.block_size % 16 == 0 &&
          k_tok == a.v_cache_stride[2] &&
          (64 % a.block_size == 0 || a.block_size % 64 == 0) && a.blocks_per_seq <= kDmaIds &&

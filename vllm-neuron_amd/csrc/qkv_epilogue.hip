@@ -470,13 +470,12 @@ int launch_qkv_epilogue(const mia_qkv_epilogue_args &a, hipStream_t s) {
   const int64_t nrows = a.num_tokens * (a.num_q_heads + 2 * a.num_kv_heads);
   if (nrows == 0) return MIA_OK;
   // groups of d/8 lanes per head row, 256 / (d/8) groups per workgroup; a
-  // workgroup takes one token and hpg heads per group: all the token's heads
-  // when there are enough tokens to fill the chip, fewer (more workgroups
-  // per token) otherwise
+  // workgroup takes hpg heads per group of one token: two when there are enough
+  // tokens to fill the chip (half the workgroups read the token's cos / sin),
+  // else one
   const int nh = a.num_q_heads + 2 * a.num_kv_heads;
   const int groups = 256 / (a.head_dim / 8);
-  const int per_wg = a.num_tokens >= 1024 ? nh : groups;
-  const int hpg = std::min(kMaxHpg, (per_wg + groups - 1) / groups);
+  const int hpg = a.num_tokens >= 1024 && nh > groups ? kMaxHpg : 1;
   const dim3 grid((unsigned)a.num_tokens, (unsigned)((nh + groups * hpg - 1) / (groups * hpg)));
   // cos / sin rows read 16 bytes at a time when contiguous and aligned
   auto al16 = [](const void *q) { return ((uintptr_t)q & 15) == 0; };
