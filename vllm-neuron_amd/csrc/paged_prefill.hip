@@ -598,10 +598,11 @@ MIA_DEV float row_max2(float x) {
 // proves that there is none, and the tile needs no maximum (16 v_max3, a lane
 // swap and a wait for all 32 scores before the first exponential).  Where a
 // sum reaches 2^8 the maximum decides, and a tile that moves it is recomputed
-// from its scores.  Results are those of testing every tile's maximum, bit for
-// bit; four-wave workgroups (777 tokens after 1536, 32 q / 8 kv heads) take
-// 51.9 us like this and 53.7 with that test.
-template <int DBLK>
+// from its scores.  BY_MAX tests every tile's maximum; both give the same bits.
+// 777 tokens after 1536 (32 q / 8 kv heads, four-wave workgroups): 51.9 us by
+// the sums, 53.7 by the maximum; the mixed batch, whose prefill shares the CUs
+// with the decode: 318.1 by the sums, 316.1 by the maximum (COMPACT below).
+template <int DBLK, bool BY_MAX = false>
 MIA_DEV float softmax_tile(f32x16_t (&sacc)[2], RowMax &rm, f32x16_t (&acc_o)[DBLK],
                            float l_run, uint32_t (&pk)[2][8]) {
   auto tile_max = [&]() {
@@ -631,6 +632,12 @@ MIA_DEV float softmax_tile(f32x16_t (&sacc)[2], RowMax &rm, f32x16_t (&acc_o)[DB
 #pragma unroll
     for (int e = 0; e < 16; ++e) rm.negm[e] = -rm.m;
   };
+  if (BY_MAX) {
+    const float mx = tile_max();
+    const bool bump = rm.set ? mx > 8.0f : mx > -INFINITY;
+    if (__builtin_amdgcn_ballot_w64(bump)) rescale(bump, mx);
+    return l_run + exp_tile(sacc, pk);
+  }
   // both tests depend on the row alone, not on the wave's other rows
   if (__builtin_expect(__builtin_amdgcn_ballot_w64(!rm.set) != 0, 0)) {
     const float mx = tile_max();
@@ -977,7 +984,10 @@ static_assert(waitcnt_vm(4) == 0xF74 && waitcnt_vm(0) == 0xF70, "vmcnt encoding"
 // Reading fragments ahead, as at d = 64, measured 2 % slower.
 // NARROW: q and out rows hold d_used < D channels; the full-width kernels test
 // nothing (the tests cost the mixed batch 0.7 %).
-template <int D, int WAVES, int STAGES, bool FP8, bool PK, int DU = D, bool NARROW = DU != D>
+// COMPACT: the launch runs beside a decode launch, whose waves fill the gaps
+// that the sum test and the V fragments read early are there for: neither.
+template <int D, int WAVES, int STAGES, bool FP8, bool PK, int DU = D, bool NARROW = DU != D,
+          bool COMPACT = false>
 __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void prefill_dma_kernel(
     PrefillKParams p) {
   static_assert(DU == D || (D == 128 && !FP8 && DU > 64 && DU % 16 == 0), "padded head dims");
@@ -997,10 +1007,11 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void prefill_dma_kernel(
   constexpr int RPI = 64 / CH;         // rows per DMA instruction
   constexpr bool AHEAD = D == 64;      // LDS operands read ahead of the products
   // key steps of V^T read before the softmax: with one wave per SIMD (4 waves)
-  // the first covers part of the LDS latency (777 tokens after 1536: 53.5 ->
-  // 52.7 us, the mixed batch's compact launch 0.4 %; two steps or K ahead: no
-  // further gain)
-  constexpr int VPRE = AHEAD ? 4 : WAVES == 4 ? 1 : 0;
+  // the first covers part of the LDS latency (777 tokens after 1536: 53.2 ->
+  // 51.9 us; two steps or K ahead: no further gain; the mixed batch with the
+  // maximum test 316.1 us without it, 317.6 with it)
+  constexpr int VPRE = AHEAD ? 4 : WAVES == 4 && !COMPACT ? 1 : 0;
+  constexpr bool BY_MAX = COMPACT;  // the rescale test of softmax_tile
   constexpr int EB = FP8 ? 1 : 2;      // cache bytes per element
   constexpr int TILE8 = kKT * D;       // bytes per FP8 K (or V) tile
   constexpr int NJ8 = 8 / kDmaWaves;   // FP8 DMA instructions per thread per tile
@@ -1249,7 +1260,7 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void prefill_dma_kernel(
       __builtin_amdgcn_sched_barrier(0);
     }
     uint32_t pk[2][8];
-    l_run = softmax_tile<DBLK>(sacc, rm, acc_o, l_run, pk);
+    l_run = softmax_tile<DBLK, BY_MAX>(sacc, rm, acc_o, l_run, pk);
 
     // ---- O^T += V^T . P^T
 #pragma unroll
@@ -2009,6 +2020,9 @@ int launch_paged_prefill(const mia_prefill_args &a, const PrefillPlan &pl, hipSt
                          s, kp);
     else if (narrow)
       hipLaunchKernelGGL((prefill_dma_kernel<128, 4, 2, false, false, 128, true>), grid,
+                         dim3(4 * 64), 0, s, kp);
+    else if (a.compact_kernel)
+      hipLaunchKernelGGL((prefill_dma_kernel<128, 4, 2, false, false, 128, false, true>), grid,
                          dim3(4 * 64), 0, s, kp);
     else
       hipLaunchKernelGGL((prefill_dma_kernel<128, 4, 2, false, false>), grid, dim3(4 * 64), 0, s,
