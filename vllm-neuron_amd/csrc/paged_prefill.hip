@@ -1758,7 +1758,7 @@ namespace {
 // Launch of one sequence.  The host knows the new tokens and, from the table's
 // width, the most keys a row tile can see.  Uncut, a short chunk after a long
 // context is a few workgroups that each walk the whole context: 200 tokens
-// after 8000 (32 q / 8 kv heads, d = 128) took 204 us on 32 of 256 CUs.
+// after 8000 (32 q / 8 kv heads, d = 128) took 206 us on 32 of 256 CUs.
 //
 // Choices: 8-wave workgroups (256 rows, one per CU) with every row tile cut
 // into n chunks, or only the row tiles left over after whole rounds of uncut
