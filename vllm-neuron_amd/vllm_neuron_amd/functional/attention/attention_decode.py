@@ -6,7 +6,8 @@ validation and error classes (:1484-1575, :1724-1741), the block-KV cache
 layout and the output layouts (:1163-1182).
 
 What runs where
-  * Up to 16 rows without a bias, stages 1 and 2 (input RMS norm, QKV
+  * Up to 16 rows without a bias, at sizes where it is faster than the
+    library (``skinny_linear_ok``), stages 1 and 2 (input RMS norm, QKV
     projection) are one HIP launch, ``mia_skinny_linear``, and stage 9 (output
     projection) another; otherwise stage 1 is the HIP row norm
     ``mia_row_norm`` and stages 2 and 9 are library GEMMs (bf16 inputs, fp32
