@@ -943,12 +943,14 @@ def _skinny_takes(x: torch.Tensor, w: torch.Tensor) -> bool:
     rows (one MFMA row block; from 17 rows on the weights would be read twice),
     whole 32-column and 32-row steps, at most 8192 columns (one workgroup of 32
     per CU).  Strides only: addresses are not known while tracing."""
-    return (x.dim() == 2 and w.dim() == 2 and x.dtype == torch.bfloat16
-            and w.dtype == torch.bfloat16 and 0 < x.shape[0] <= 16 and x.shape[1] == w.shape[0]
-            and x.shape[1] % 32 == 0 and w.shape[1] % 32 == 0 and 0 < w.shape[1] <= 8192
-            and x.shape[1] > 0 and x.stride(1) == 1
-            and w.stride(1) == 1 and x.stride(0) % 8 == 0 and w.stride(0) % 2 == 0
-            and w.stride(0) >= w.shape[1] and (x.shape[0] == 1 or x.stride(0) >= x.shape[1]))
+    if (x.dim() != 2 or w.dim() != 2 or x.dtype != torch.bfloat16
+            or w.dtype != torch.bfloat16):
+        return False
+    (T, k), (wk, n) = x.shape, w.shape
+    (xs, xc), (ws, wc) = x.stride(), w.stride()
+    return (0 < T <= 16 and k == wk and k > 0 and k % 32 == 0 and n % 32 == 0 and 0 < n <= 8192
+            and xc == 1 and wc == 1 and xs % 8 == 0 and ws % 2 == 0 and ws >= n
+            and (T == 1 or xs >= k))
 
 
 def skinny_linear_ok(x: torch.Tensor, w: torch.Tensor) -> bool:

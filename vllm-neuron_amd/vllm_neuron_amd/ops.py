@@ -536,9 +536,10 @@ def skinny_linear_ok(x: Tensor, w: Tensor) -> bool:
     if not K.skinny_linear_ok(x, w) or (torch.is_grad_enabled()
                                         and (x.requires_grad or w.requires_grad)):
         return False
-    dev = x.device.type
-    if torch.is_autocast_enabled(dev) and torch.get_autocast_dtype(dev) != torch.bfloat16:
-        return False
+    if torch._C._is_any_autocast_enabled():
+        dev = x.device.type
+        if torch.is_autocast_enabled(dev) and torch.get_autocast_dtype(dev) != torch.bfloat16:
+            return False
     if torch.compiler.is_compiling():  # traced: x and w are plain tensors there
         return True
     return (forward_ad._current_level < 0 and not torch._C._are_functorch_transforms_active()
